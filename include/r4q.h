@@ -389,13 +389,12 @@ R4Q_API int r4q_decode_profile(r4q_ctx* ctx, const r4q_model* m, const void* hid
  * choice).  Knobs: "gemv_lpr" (lanes per GEMV row: 16..256, power of two),
  * "gemv_wgs" (GEMV workgroup cap, 1..65536), "gemv_ub" (GEMV steps in flight
  * per lane, 1..2), "attn_splits" (flash-decode splits, 1..128), "skinny_splits"
- * (skinny GEMM K splits, 1..8), "gemm_splits" (ring GEMM: 1 = whole tiles
+ * (skinny GEMM K splits, 1..8), "gemm_splits" (tile GEMM: 1 = whole tiles
  * only, 2..16 = stream-K with about that many workgroups per tile),
  * "split_reduce" (1 = batched decode steps reduce the split-K partials of
  * the qkv, o and down projections in their own launches, not in the
- * attention prologue / row norm that consume them), "gemm_kernel" (GEMM for
- * M >= 256: 1 = the ring kernel (the default), 2 = the specialised-wave
- * kernel where it applies: INT4, N % 128 == 0, K % 256 == 0), "gemv_skew"
+ * attention prologue / row norm that consume them), "gemm_kernel" (1 or 2,
+ * without effect: one kernel serves every M > 16), "gemv_skew"
  * (GEMV on an even grid of more than 256 equal shares: the first half of the
  * workgroups takes value - 1 steps more and the second half value - 1 fewer;
  * 1 = equal shares; default 2 on a 512-workgroup grid of at least 4 steps

@@ -43,11 +43,8 @@ int gemv_fwht_launch(const void* x16, const float* h, int64_t split, const void*
 constexpr int64_t kSkinnyMaxRows = 16;
 
 // MFMA GEMM (r4q_gemm.hip), arguments validated by the caller.  ws
-// (ws_bytes of device memory, may be null) holds the fp32 partials of a
-// split-K launch; gemm_splits() gives the split count a workspace allows
-// (1: none needed).
-constexpr int kMaxGemmSplits = 16;
-int gemm_splits(int64_t M, int64_t N, int64_t K, int wbits, size_t ws_bytes);
+// (ws_bytes of device memory, may be null) holds the partials of a split-K
+// launch.
 // Workspace bytes for the best split count of a shape (0: none needed).
 size_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int wbits);
 int gemm_mfma_launch(const void* x, const void* w, const void* sz, void* y, int64_t M, int64_t N,

@@ -29,10 +29,8 @@ int launch_status(const char* what);
 //   gemv_ub       R4Q_GEMV_UB       GEMV steps in flight per lane: 1 or 2
 //   attn_splits   R4Q_ATTN_SPLITS   flash-decode splits: 1 .. 128
 //   skinny_splits R4Q_SKINNY_SPLITS skinny-GEMM K splits: 1 .. 8
-//   gemm_splits   R4Q_GEMM_SPLITS   ring GEMM: 1 whole tiles, 2 .. 16 stream-K workgroups per tile
-//   gemm_kernel   R4Q_GEMM_KERNEL   GEMM for M >= 256: 1 the ring kernel (the default), 2 the
-//                                   specialised-wave kernel where it applies (INT4, N % 128 == 0,
-//                                   K % 256 == 0)
+//   gemm_splits   R4Q_GEMM_SPLITS   tile GEMM: 1 whole tiles, 2 .. 16 stream-K workgroups per tile
+//   gemm_kernel   R4Q_GEMM_KERNEL   1 or 2, without effect: one kernel serves every M > 16
 //   gemv_skew     R4Q_GEMV_SKEW     GEMV on an even grid of more than 256 equal shares: the
 //                                   first half takes value - 1 steps more, the second half
 //                                   value - 1 fewer (1 = equal shares)

@@ -354,3 +354,64 @@ def test_spec_gemm_one_hot_columns_exact(dev, splits):
         R.tune("gemm_splits", 0)
     for r, k in enumerate(ks):
         assert np.array_equal(y[r], W[:, k]), (r, k)
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16])
+@pytest.mark.parametrize("M,N,K", [(17, 131, 32), (32, 128, 160), (33, 260, 1056), (64, 129, 4128),
+                                   (65, 640, 2080), (96, 127, 224), (97, 513, 4096),
+                                   (128, 20000, 96), (129, 1000, 1312), (255, 383, 4192),
+                                   (256, 257, 1056), (257, 70, 96), (513, 1030, 2080)])
+def test_tile_gemm_edges(dev, bits, M, N, K):
+    """M > 16: one row past and one short of every tile height, widths off the
+    tile and off the 16-byte store, K shorter than a step and ending inside one,
+    split and unsplit (no workspace).  The fp16 output rounds within 2^-12
+    relative (rel-L2 below 2.9e-4), a fp16 partial (M >= 256) as much again per
+    segment: 1e-3 is twice their sum over the at most 16 segments' random
+    signs.  Below 256 rows an output is one chain over k in any tile, so rows
+    alone in a smaller tile (their first 17) give the same bits."""
+    import r4q_lib as R
+    g = S.gen(M + 7 * N + K + bits)
+    w, sz = S.weight(N, K, bits, g)
+    x = torch.randn(M, K, generator=g).half()
+    X, Wd, SZ = x.to(dev), w.to(dev), None if sz is None else sz.to(dev)
+    want = _ref32(x, w, sz, bits)
+    split = int4_hip.dbg_gemm(X, Wd, SZ, M, N, K)
+    whole = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+    R.call("r4q_gemm", X.data_ptr(), Wd.data_ptr(), None if SZ is None else SZ.data_ptr(),
+           whole.data_ptr(), M, N, K, bits, R.stream_handle())
+    for y in (split, whole):
+        got = y.float().cpu().numpy()
+        assert np.all(np.isfinite(got))
+        assert rel_l2(got, want) <= 1e-3
+        for r in (0, M // 2, M - 1):
+            assert rel_l2(got[r], want[r]) <= 1e-3, r
+    few = int4_hip.dbg_gemm(X[:17].contiguous(), Wd, SZ, 17, N, K)
+    assert torch.equal(few.view(torch.int16), whole[:17].view(torch.int16))
+    if M < 256:
+        assert torch.equal(split.view(torch.int16), whole.view(torch.int16))
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16])
+@pytest.mark.parametrize("M,N,K", [(40, 200, 288), (120, 150, 2080), (260, 300, 352)])
+def test_tile_gemm_one_hot_and_infinite_rows(dev, bits, M, N, K):
+    """Row r of x = e_k(r) gives column k(r) of the dequantised weight bit for
+    bit, K ending inside a step; an infinity in the row's last element reaches
+    only its own row and, times a non-zero weight, stays an infinity (a step
+    past K multiplies zeros, not the repeated last elements)."""
+    g = S.gen(5 * M + N + K + bits)
+    w, sz = S.weight(N, K, bits, g)
+    W = O.dequant(w.numpy(), None if sz is None else sz.numpy(), bits)
+    ks = [(r * 97 + r // 3) % K for r in range(M)]
+    ks[1] = K - 1
+    x = torch.zeros(M, K, dtype=torch.float16)
+    for r, k in enumerate(ks):
+        x[r, k] = 1.0
+    x[2, :] = 0.0
+    x[2, K - 1] = float("inf")
+    y = int4_hip.dbg_gemm(x.to(dev), w.to(dev), None if sz is None else sz.to(dev), M, N, K)
+    y = y.cpu().numpy()
+    for r, k in enumerate(ks):
+        if r != 2:
+            assert np.array_equal(y[r], W[:, k]), (r, k)
+    nz = W[:, K - 1] != 0
+    assert np.array_equal(y[2][nz], np.where(W[nz, K - 1] > 0, np.inf, -np.inf).astype(np.float16))
