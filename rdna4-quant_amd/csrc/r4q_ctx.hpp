@@ -35,8 +35,7 @@ struct r4q_ctx {
   void* tail_zeroed = nullptr;  // batched gate/up tail counters known to be zero
   r4q::DevBuf prefill;   // prefill activations
   r4q::DevBuf misc;      // device-side position / counters
-  r4q::DevBuf sample;    // sampling tables (kept zeroed between calls)
-  size_t sample_zeroed = 0;  // bytes of `sample` known to be zero
+  r4q::DevBuf sample;    // sampling tables
   r4q::GraphCache* graphs = nullptr;
   r4q_ctx() {
     for (r4q::DevBuf* b : {&attn, &step, &prefill, &misc, &sample}) b->epoch = &buf_epoch;
@@ -48,8 +47,8 @@ namespace r4q {
 // Flash-decode internals used by the decode step.
 // Chooses the split count for `seq_len` positions over B*Hk heads.
 int attn_num_splits(int64_t seq_len, int64_t B, int64_t Hk);
-// Sampling workspace for B rows, zeroed on (re)allocation.
-int sample_reserve(r4q_ctx* ctx, int64_t B, hipStream_t st, void** ws);
+// Sampling workspace for B rows.
+int sample_reserve(r4q_ctx* ctx, int64_t B, void** ws);
 // Bytes of partial-result scratch for a launch.
 size_t attn_ws_bytes(int64_t B, int64_t H, int nsplit);
 // Enqueues partial + combine; seq_len_dev != nullptr: length read on device

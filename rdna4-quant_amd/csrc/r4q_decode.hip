@@ -823,7 +823,7 @@ int decode_loop(r4q_ctx* ctx, const r4q_model* m, const void* hidden_in, int64_t
   R4Q_TRY(reserve(ctx, m, dm, B, nsplit, st, bf));
   int64_t* toks = static_cast<int64_t*>(tokens_out);
   void* sws = nullptr;
-  if (scfg.temperature > 0.f) R4Q_TRY(sample_reserve(ctx, B, st, &sws));
+  if (scfg.temperature > 0.f) R4Q_TRY(sample_reserve(ctx, B, &sws));
   const size_t hbytes = (size_t)B * dm.D * 2;
   if (!use_graph) {
     R4Q_HIP_TRY(hipMemcpyAsync(bf.h, hidden_in, hbytes, hipMemcpyDeviceToDevice, st));

@@ -43,8 +43,8 @@ struct SampleCfg {
   float top_p;
   uint64_t seed;
 };
-// Workspace for B <= 1024 rows: the selection words, then a zeroed
-// 65,536-bin table per row (left zeroed by every call; see sample_reserve).
+// Workspace for B <= 1024 rows: the selection words, then a 65,536-bin table
+// per row (written whole by every call).
 size_t sample_ws_bytes(int64_t B);
 // ids[b] = sampled token of row b of logits [B, stride] fp16 (V used).
 // counter_dev (device int) overrides counter_host.  With embed != nullptr

@@ -136,3 +136,25 @@ def test_sampled_decode_loop_eager_graph_and_host(dev):
         tok = int(int4_hip.sample(lg.reshape(-1), T, top_p, seed, 10 + t).item())
         assert tok == int(toks_e[t]), t
         hid = m.embed_d[tok].view(1, 1, m.D).contiguous()
+
+
+@pytest.mark.parametrize("V", [1, 7, 9, 511, 513, 8191, 8193, 16385, 151935])
+@pytest.mark.parametrize("offset", [0, 1, 5])
+def test_sample_odd_rows_and_ties(dev, V, offset):
+    """Rows of any length at any 2-byte offset (the kernels read 16-byte groups
+    of aligned rows): greedy picks the first maximum; among rows of one repeated
+    value a draw u takes token floor(u V) of the tied bin, whichever wave's part
+    of the row holds it."""
+    flat = torch.full((3 * V + offset + 8,), 1.5, dtype=torch.float16, device=dev)
+    rows = flat[offset:offset + 3 * V].view(3, V)
+    got = int4_hip.sample(rows, 1.0, 1.0, 7, 11).cpu().tolist()
+    for b in range(3):
+        u = O.sample_uniform(7, 11, b)
+        want = min(int(np.floor(np.float32(u) * np.float32(V))), V - 1)
+        assert abs(got[b] - want) <= max(1, int(V * MARGIN)), (b, got[b], want)
+    x = torch.stack([_logits(V, 5 * V + offset + b, ties=False) for b in range(3)])
+    x[1, V - 1] = x[1].max()
+    x[2, V // 2:] = x[2].max()
+    rows.copy_(x.to(dev))
+    want = [int(np.argmax(r.float().numpy())) for r in x]  # the first maximum
+    assert int4_hip.sample(rows, 0.0).cpu().tolist() == want
