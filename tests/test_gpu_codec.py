@@ -69,6 +69,34 @@ def test_dequant_int8_bit_exact(dev, N, K):
     assert np.array_equal(got.view(np.uint16), want.view(np.uint16))
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 1023, 1024, 1025, 8191, 8192, 8193, 16397])
+def test_fp8_codecs_at_every_alignment(dev, n):
+    """Whole and partial turns of a workgroup, with the source at each
+    alignment the entry points take: 8 bytes for fp16, 1 for codes."""
+    bits = (np.arange(n + 8, dtype=np.uint32) * 40503 + n).astype(np.uint16)
+    x = torch.from_numpy(bits.view(np.int16)).view(torch.float16).to(dev)
+    codes = torch.from_numpy((bits >> 3).astype(np.uint8)).to(dev)
+    for off in (0, 4, 8):
+        got = int4_hip.fp16_to_fp8(x[off:off + n]).cpu().numpy()
+        assert np.array_equal(got, fp8_golden_table()[bits[off:off + n]])
+    for off in (0, 1, 4, 8):
+        got = int4_hip.fp8_to_fp16(codes[off:off + n]).cpu().double().numpy()
+        want = O.fp8_value((bits[off:off + n] >> 3).astype(np.uint8))
+        ok = ~np.isnan(want)
+        assert np.array_equal(got[ok], want[ok])
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,K", [(1, 32), (1, 8160), (1, 8192), (255, 32), (257, 64), (3, 8224)])
+def test_dequant_turn_edges(dev, bits, N, K):
+    g = S.gen(N + K + bits)
+    w, sz = (S.int4_weight if bits == 4 else S.int8_weight)(N, K, g)
+    f, o = ((int4_hip.dequant_int4, O.dequant_int4) if bits == 4
+            else (int4_hip.dequant_int8, O.dequant_int8))
+    got = f(w.to(dev), sz.to(dev), N, K).cpu().numpy()
+    assert np.array_equal(got.view(np.uint16), o(w.numpy(), sz.numpy()).view(np.uint16))
+
+
 def test_dequant_rejects_bad_shape(dev):
     w = torch.zeros(4, 24, dtype=torch.uint8, device=dev)
     s = torch.zeros(4, 3, dtype=torch.float16, device=dev)
