@@ -154,9 +154,10 @@ __device__ __forceinline__ uint32_t pk_add_h(uint32_t a, uint32_t b) {  // fp16 
   return r;
 }
 __device__ __forceinline__ uint32_t cvt_pk_h(float lo, float hi) {  // (fp16(lo), fp16(hi))
-  uint32_t r;
-  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
-  return r;
+  typedef float f2_t __attribute__((ext_vector_type(2)));
+  // not inline assembly: an operand that v_exp_f32 wrote just before needs a wait
+  // state, which the compiler only inserts for instructions it knows
+  return as_u32(__builtin_convertvector((f2_t{lo, hi}), h2_t));
 }
 
 __device__ __forceinline__ void load16w(const uint16_t* __restrict__ p, uint32_t* w) {

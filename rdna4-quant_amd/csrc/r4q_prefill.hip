@@ -33,40 +33,103 @@ __global__ __launch_bounds__(256) void embed_gather_kernel(const int64_t* __rest
 // heads at h*128, k heads at (H + kh)*128 and v heads at (H + Hk + kh)*128,
 // kh = h / (H/Hk).  out[m, h*128 + d] =
 //   FWHT32(softmax_{j <= m}(q_m . k_j / sqrt(128)) V)[d].
-// Keys go in blocks of 32 through LDS (K row-major, V transposed), the next
-// block's global loads in flight during the current block's arithmetic.
+// Keys go in blocks of 32 through LDS, two stages each for K and for V filled by
+// direct copies.  Both tiles are row major, 256 bytes a key, the 16-byte pieces of
+// row r at piece ^ (r & 15) for K and piece ^ 2 (r & 7) for V, which spreads each
+// read below over all banks.  In turn kb a wave takes S of block kb + 1 (matrix
+// cores) and the softmax and P V of block kb, two chains that do not depend on
+// each other; K of kb + 2 and V of kb + 1 are in flight.
 // Per block and wave (lane l: column n = l % 16, group g = l / 16):
 //  * S^T = K Q^T for two 16-key halves: A = K (lane: key n of the half,
 //    dims 32k + 8g .. over the 4 k-steps), B = Q^T (lane: query row n, the
 //    same dims, held in registers for the whole loop).  C: lane holds query
 //    n at keys 4g .. 4g+3 of the half;
 //  * online softmax per query across the 4 lanes holding it, probabilities
-//    rounded to fp16, keys past the query (or the prompt) masked;
+//    rounded to fp16, keys past the query masked (in the diagonal block only);
 //  * O += P V: A = P (lane: query n; k-slots = its 8 keys 4g + r and
-//    16 + 4g + r), B = V (lane: dim 16j + n of N-block j, the same keys,
-//    two 8-byte reads of the transposed block).  C: lane holds dim 16j + n
-//    of queries 4g .. 4g+3.
+//    16 + 4g + r), B = V (lane: dim 16j + n of N-block j, the same keys: two
+//    transposing LDS reads).  C: lane holds dim 16j + n of queries 4g .. 4g+3.
+//    O is rescaled only where some row's maximum moved (a factor of 1 is exact).
 // Epilogue: O / l, FWHT-32 per 32-dim chunk (the 16-dim step inside the
 // lane, steps 1 .. 8 across lanes xor 1 .. 8), one fp16 rounding.
-constexpr int kFaKRow = 136;  // halves per K row in LDS (128 + 8 pad)
-constexpr int kFaVRow = 36;   // halves per transposed-V row (32 keys + 4 pad)
+//
+// Bound by the softmax's vector instructions with the waves that one CU holds (four
+// workgroups, 128 VGPRs).  40 heads over 8 K/V heads, 2000 rows: 207 -> 82 us; 512
+// rows: 31 -> 19 us, a chain of 16 turns in the longest workgroup.  Before, V was
+// transposed by 2-byte LDS stores that conflicted 4 ways, K, softmax and V of a
+// block were one chain, and the tiles with the fewest keys came first.  32 query
+// rows per wave (half the LDS reads per row) measured 93 and 27 us.
+constexpr int kFaRows = 64;        // query rows of a workgroup
+constexpr int kFaTile = 32 * 256;  // bytes of a block's K (or V) in LDS: K, K, V, V
 
-__global__ __launch_bounds__(256) void prefill_fa_kernel(const uint16_t* __restrict__ qkv,
-                                                         int64_t stride,
-                                                         uint16_t* __restrict__ out,
-                                                         int64_t out_stride, int M, int H,
-                                                         int Hk) {
-  __shared__ __align__(16) uint16_t ks[32 * kFaKRow];
-  __shared__ __align__(16) uint16_t vt[128 * kFaVRow];
-  const int h = blockIdx.x, q0 = blockIdx.y * 64;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+typedef __attribute__((address_space(3))) uint8_t lds8;
+typedef short s4_t __attribute__((ext_vector_type(4)));
+
+// Global -> LDS copy of 16 bytes per lane (lane l's land at lds + 16 l), as inline
+// assembly so that the compiler does not wait for it before unrelated LDS reads:
+// the kernel waits for its own copies.
+__device__ __forceinline__ void copy16(const void* src, lds8* lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(
+                   __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds)),
+               "v"(src)
+               : "memory");
+}
+
+// maximum over the lanes n, n + 16, n + 32, n + 48, in all of them
+__device__ __forceinline__ float max_groups(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  const uint32_t w = __builtin_bit_cast(uint32_t, v);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]),
+               __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
+__global__ __launch_bounds__(256, 4) void prefill_fa_kernel(const uint16_t* __restrict__ qkv,
+                                                            int64_t stride,
+                                                            uint16_t* __restrict__ out,
+                                                            int64_t out_stride, int M, int H,
+                                                            int Hk) {
+  __shared__ __align__(1024) uint8_t smem[4 * kFaTile];
+  lds8* const lds = (lds8*)smem;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int col = lane & 15, g = lane >> 4;
+  // workgroup -> (head, query tile): the tiles with the most keys first, and a
+  // run of heads (which share K/V heads) per XCD where the head count allows
+  int h, qt;
+  {
+    const int S = H % 8 == 0 ? 8 : 1, id = blockIdx.x, j = id / S, hc = H / S;
+    h = (id % S) * hc + j % hc;
+    qt = (int)(gridDim.x / H) - 1 - j / hc;
+  }
+  const int q0 = qt * kFaRows;
   const int kh = h / (H / Hk);
   const uint16_t* kbase = qkv + (int64_t)(H + kh) * 128;
-  const uint16_t* vbase = qkv + (int64_t)(H + Hk + kh) * 128;
-  const int r0 = q0 + 16 * wave;  // this wave's first query row
-  const int kend = min(q0 + 64, M);  // the workgroup needs keys [0, kend)
-  const int nkb = (kend + 31) / 32;
+  const int r0 = q0 + 16 * wave;                     // this wave's first query row
+  const int nkb = (min(q0 + kFaRows, M) + 31) / 32;  // blocks of keys of the workgroup
+  const int nwb = min(nkb, r0 / 32 + 1);             // and of this wave; the last one masked
+
+  // staging: 512 16-byte slots per tile (slot 16 row + place), two copies per
+  // thread, the source pieces swizzled as above; keys past the prompt clamped.
+  // kp, vp: this thread's first piece of the next K and V block to load
+  const int srow = 4 * wave + g;
+  const uint16_t* kp = kbase + srow * stride + 8 * (col ^ srow);
+  const uint16_t* vp = kbase + Hk * 128 + srow * stride + 8 * (col ^ (2 * (srow & 7)));
+  auto load_tile = [&](const uint16_t*& p, int kb, int tile) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint16_t* src = p + 16 * i * stride;
+      if (32 * kb + 32 > M)  // rows past the prompt: its last one
+        src -= max(32 * kb + 16 * i + srow - (M - 1), 0) * stride;
+      copy16(src, lds + tile * kFaTile + 4096 * i + 1024 * wave);
+    }
+    p += 32 * stride;
+  };
+  load_tile(kp, 0, 0);
+  load_tile(vp, 0, 2);
+  if (nkb > 1) load_tile(kp, 1, 1);
 
   // Q^T fragments: qb[k] = Q[row r0 + col][32k + 8g .. +7] (rows past M clamped)
   u4_t qb[4];
@@ -75,71 +138,54 @@ __global__ __launch_bounds__(256) void prefill_fa_kernel(const uint16_t* __restr
 #pragma unroll
     for (int k = 0; k < 4; ++k) qb[k] = *reinterpret_cast<const u4_t*>(qr + 32 * k);
   }
-  // block staging: piece t and t + 256 of 512 16-byte pieces (key t / 16,
-  // dims 8 (t % 16) ..) for K and for V; keys past the prompt clamped
-  u4_t kp[2], vp[2];
-  auto load_block = [&](int kb) {
+  int ka[4], va[4];  // LDS offsets of the reads: stage 0, first 16 keys, j < 4
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int pc = t + 256 * i, key = min(32 * kb + (pc >> 4), M - 1), d8 = 8 * (pc & 15);
-      kp[i] = *reinterpret_cast<const u4_t*>(kbase + (int64_t)key * stride + d8);
-      vp[i] = *reinterpret_cast<const u4_t*>(vbase + (int64_t)key * stride + d8);
-    }
-  };
-  auto store_block = [&]() {
+  for (int k = 0; k < 4; ++k) ka[k] = 256 * col + 16 * ((4 * k + g) ^ col);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int pc = t + 256 * i, key = pc >> 4, d8 = 8 * (pc & 15);
-      *reinterpret_cast<u4_t*>(ks + key * kFaKRow + d8) = kp[i];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        vt[(d8 + 2 * e) * kFaVRow + key] = (uint16_t)(vp[i][e] & 0xFFFFu);
-        vt[(d8 + 2 * e + 1) * kFaVRow + key] = (uint16_t)(vp[i][e] >> 16);
-      }
-    }
-  };
+  for (int j = 0; j < 4; ++j) {
+    const int row = 4 * g + (col >> 2);
+    va[j] = 2 * kFaTile + 256 * row + 16 * ((2 * j + ((col & 3) >> 1)) ^ (2 * (row & 7))) +
+            8 * (col & 1);
+  }
 
   const float sscale = 0.08838834764831845f;  // 1 / sqrt(128)
   const uint32_t ones = 0x3C003C00u;           // fp16 (1, 1)
   float m_run = -INFINITY, l_run = 0.f;        // query col; l over this lane's keys
-  f4_t o[8];
+  f4_t o[8], s0[2], s1[2];                      // s0, s1: scores of even and odd blocks
 #pragma unroll
   for (int j = 0; j < 8; ++j) o[j] = f4_t{0.f, 0.f, 0.f, 0.f};
-  auto kpos = [&](int s) { return s < 4 ? 4 * g + s : 16 + 4 * g + (s - 4); };
+  auto kpos = [&](int e) { return e < 4 ? 4 * g + e : 16 + 4 * g + (e - 4); };
 
-  load_block(0);
-  for (int kb = 0; kb < nkb; ++kb) {
-    __syncthreads();  // the previous block's LDS reads are done
-    store_block();
-    __syncthreads();
-    if (kb + 1 < nkb) load_block(kb + 1);  // in flight during this block
-    if (32 * kb > r0 + 15) continue;       // wave-uniform: block entirely past this wave's rows
-    // ---- S^T = K Q^T
-    f4_t sacc[2];
+  // S^T = K Q^T of the block in K stage `stage`
+  auto scores = [&](f4_t(&s)[2], int stage) {
 #pragma unroll
     for (int bb = 0; bb < 2; ++bb) {
-      sacc[bb] = f4_t{0.f, 0.f, 0.f, 0.f};
-      const uint16_t* kr = ks + (16 * bb + col) * kFaKRow + 8 * g;
+      s[bb] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        sacc[bb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            __builtin_bit_cast(h8_t, *reinterpret_cast<const u4_t*>(kr + 32 * k)),
-            __builtin_bit_cast(h8_t, qb[k]), sacc[bb], 0, 0, 0);
+      for (int k = 0; k < 4; ++k) {
+        const h8_t kf = *(const __attribute__((address_space(3))) h8_t*)(lds + ka[k] + 4096 * bb +
+                                                                         stage * kFaTile);
+        s[bb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, __builtin_bit_cast(h8_t, qb[k]), s[bb],
+                                                       0, 0, 0);
+      }
     }
-    // ---- online softmax for query r0 + col over keys 32 kb + kpos(s)
-    const int qabs = r0 + col;
+  };
+  // online softmax for query r0 + col over block kb's keys 32 kb + kpos(e), O += P V
+  auto attend = [&](const f4_t(&s)[2], int kb, int stage, bool masked) {
+    // scores are rounded before the maximum is subtracted, in every block alike
+#pragma clang fp contract(off)
     float sv[8];
 #pragma unroll
-    for (int s = 0; s < 8; ++s)
-      sv[s] = (32 * kb + kpos(s) <= qabs) ? sacc[s >> 2][s & 3] * sscale : -INFINITY;
+    for (int e = 0; e < 8; ++e) {
+      sv[e] = s[e >> 2][e & 3] * sscale;
+      if (masked && 32 * kb + kpos(e) > r0 + col) sv[e] = -INFINITY;
+    }
     float mx = sv[0];
 #pragma unroll
-    for (int s = 1; s < 8; ++s) mx = fmaxf(mx, sv[s]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float mn = fmaxf(m_run, mx);  // finite: key 32 kb <= r0 <= qabs is unmasked
-    const float alpha = (m_run == -INFINITY) ? 0.f : __expf(m_run - mn);
-    u4_t pa;  // fp16 probabilities, k-slot s = key kpos(s)
+    for (int e = 1; e < 8; ++e) mx = fmaxf(mx, sv[e]);
+    const float mn = fmaxf(m_run, max_groups(mx));  // finite: key 32 kb is unmasked
+    const float alpha = __expf(m_run - mn);         // 0 in the first block
+    u4_t pa;                                        // fp16 probabilities, k-slot e = key kpos(e)
     float lp = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -149,22 +195,55 @@ __global__ __launch_bounds__(256) void prefill_fa_kernel(const uint16_t* __restr
     }
     l_run = __builtin_fmaf(l_run, alpha, lp);
     m_run = mn;
-    float ar[4];  // alpha of the C rows' queries 4g + r (lane 4g + r holds that query)
+    if (__any(!(alpha == 1.0f))) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * g + r);
-    // ---- O += P V
+      for (int r = 0; r < 4; ++r) {  // query 4g + r of C's rows: lane 4g + r holds its alpha
+        const float ar = __shfl(alpha, 4 * g + r);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j][r] *= ar;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const uint16_t* vr = vt + (16 * j + col) * kFaVRow + 4 * g;
-      const u2_t lo = *reinterpret_cast<const u2_t*>(vr);
-      const u2_t hi = *reinterpret_cast<const u2_t*>(vr + 16);
-      const u4_t vb = u4_t{lo[0], lo[1], hi[0], hi[1]};
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[j][r] *= ar[r];
-      o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, pa),
-                                                    __builtin_bit_cast(h8_t, vb), o[j], 0, 0, 0);
+      typedef __attribute__((address_space(3))) s4_t lds_s4;
+      lds8* const v = lds + (va[j & 3] ^ (j < 4 ? 0 : 128)) + stage * kFaTile;
+      const u2_t lo = __builtin_bit_cast(u2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)v));
+      const u2_t hi =
+          __builtin_bit_cast(u2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(v + 4096)));
+      const h8_t vb = __builtin_bit_cast(h8_t, (u4_t{lo[0], lo[1], hi[0], hi[1]}));
+      o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, pa), vb, o[j], 0, 0,
+                                                    0);
     }
+  };
+  // this wave's copies so far have landed, after the barrier everyone's, and
+  // everyone's LDS reads of the turn before are done
+  auto sync = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  auto begin = [&](int kb, int st) {  // st = kb & 1
+    sync();
+    if (kb + 2 < nkb) load_tile(kp, kb + 2, st);
+    if (kb + 1 < nkb) load_tile(vp, kb + 1, 3 - st);
+  };
+  sync();
+  scores(s0, 0);
+  int kb = 0;
+  for (; kb + 2 < nwb; kb += 2) {
+    begin(kb, 0);
+    scores(s1, 1);
+    attend(s0, kb, 0, false);
+    begin(kb + 1, 1);
+    scores(s0, 0);
+    attend(s1, kb + 1, 1, false);
   }
+  begin(kb, 0);
+  if (kb + 1 < nwb) {
+    scores(s1, 1);
+    attend(s0, kb, 0, false);
+    begin(++kb, 1);
+    s0[0] = s1[0];
+    s0[1] = s1[1];
+  }
+  attend(s0, kb, kb & 1, true);
+  for (++kb; kb < nkb; ++kb) begin(kb, kb & 1);  // the other waves' last blocks
   // ---- O / l, FWHT-32, fp16 out (rows 4g + r of the wave's 16)
   float lsum = l_run + __shfl_xor(l_run, 16);
   lsum += __shfl_xor(lsum, 32);
@@ -215,8 +294,8 @@ int launch_embed_gather(const int64_t* ids, const void* table, void* out, int64_
 int launch_prefill_attention(const void* qkv, int64_t stride, void* out, int64_t out_stride,
                              int64_t M, int64_t H, int64_t Hk, hipStream_t st) {
   if (M == 0) return R4Q_OK;
-  hipLaunchKernelGGL(prefill_fa_kernel, dim3((unsigned)H, (unsigned)((M + 63) / 64)), dim3(256),
-                     0, st, static_cast<const uint16_t*>(qkv), stride,
+  hipLaunchKernelGGL(prefill_fa_kernel, dim3((unsigned)(H * ((M + kFaRows - 1) / kFaRows))),
+                     dim3(256), 0, st, static_cast<const uint16_t*>(qkv), stride,
                      static_cast<uint16_t*>(out), out_stride, (int)M, (int)H, (int)Hk);
   return launch_status("prefill_attention");
 }

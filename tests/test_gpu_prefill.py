@@ -134,3 +134,29 @@ def test_prefill_attention_vs_oracle(dev, M, H, Hk):
     assert rel_l2(got, want) <= TOL
     for r in sorted({0, M // 2, M - 1}):
         assert rel_l2(got[r], want[r]) <= TOL, r
+
+
+@pytest.mark.parametrize("trend", ["rising", "falling", "flat"])
+@pytest.mark.parametrize("M", [33, 95, 97, 160, 321])
+def test_prefill_attention_score_trends(dev, M, trend):
+    """Scores that move every row's maximum in each 32-key block, only in the
+    first, or never (all equal), over whole and partial blocks and tiles; 8
+    heads (one per XCD) and 3."""
+    import r4q_lib as R
+    for H, Hk in ((8, 4), (3, 1)):
+        g = torch.Generator().manual_seed(M + H)
+        n = (H + 2 * Hk) * 128
+        qkv = torch.randn(M, n, generator=g).half()
+        slope = {"rising": 1.0, "falling": -1.0, "flat": 0.0}[trend]
+        qkv[:, :H * 128] = 1.0  # score of key j = slope 0.05 sqrt(128) j
+        qkv[:, H * 128:(H + Hk) * 128] = (slope * 0.05 * torch.arange(M).float())[:, None].half()
+        q, k, v = qkv.split([H * 128, Hk * 128, Hk * 128], 1)
+        want = O.attention_prefill(q.reshape(M, H, 128).numpy(), k.reshape(M, Hk, 128).numpy(),
+                                   v.reshape(M, Hk, 128).numpy(), H, Hk, fwht=True)
+        out = torch.empty(M, H * 128, dtype=torch.float16, device=dev)
+        R.call("r4q_prefill_attention", qkv.to(dev).data_ptr(), n, out.data_ptr(), H * 128, M, H,
+               Hk, R.stream_handle())
+        got = out.cpu().numpy()
+        assert np.all(np.isfinite(got))
+        for r in {0, 31, 32, M // 2, M - 1}:
+            assert rel_l2(got[r], want[r]) <= TOL, r
