@@ -15,7 +15,9 @@
  *   FP16 weight  w  [N, K]    fp16
  *   scale/zero  sz  [N, K/32, 2] fp16, interleaved (scale, zero-point) per
  *                              32-element block; unused for FP16 weights.
- *   dequantised weight = fp16( (float(q) - float(zp)) * float(scale) )
+ *   dequantised weight = fp16( (float(q) - float(zp)) * float(scale) );
+ *   the GEMM over 2..16 and over 256 and more rows takes zero-points as whole
+ *   numbers (0..1024, what checkpoints hold) and rounds others to them.
  *   FP8 KV cache [B, Hk, max_seq, head_dim] uint8, E4M3 codes written by the
  *   reference recipe (see r4q_fp16_to_fp8), optional per-head fp32 scale:
  *   stored = fp8(value * (1/scale)), read back as fp8_value * scale.

@@ -15,8 +15,10 @@
 //    a caller workspace);
 //  * gemm_skinny_kernel (2 <= M <= 16): weights streamed once for all rows
 //    through an LDS ring (split along K for narrow N).
-// Dequantised values equal r4q_dequant_int4/8 bit-for-bit
-// (fp16((q - zp) * scale) from an exact product, one rounding).
+// Dequantised values equal r4q_dequant_int4/8 bit-for-bit (fp16((q - zp) * scale)
+// from an exact product, one rounding): between 17 and 255 rows for every
+// zero-point, elsewhere for whole numbers up to 1024 (others are rounded to the
+// nearest one: zp + 1024 is a fp16 number there).
 #include <stdint.h>
 #include <stdlib.h>
 
@@ -221,6 +223,7 @@ struct Tile {
 template <int WBITS, int MT, int NF, int MG>
 struct TileSeg {
   using T = Tile<WBITS, MT, NF, MG>;
+  static constexpr bool kAnyZp = MG == 1 && WBITS != 16;  // exact for every zero-point
   lds8* ring;
   const uint8_t *X, *W, *SZ;  // first row of the tile
   int K, ka, ke, nk, wave, col, g, mg, ws;  // k range [ka, ke) in nk steps
@@ -372,9 +375,10 @@ struct TileSeg {
   }
 
   // Pair k (labels 2k, 2k + 1) of B fragment f of MFMA k-step j: fp16((q - zp)
-  // * scale), bit-identical to the dequant kernel (as dq_pair).  One pair at a
-  // time, so that the arithmetic can be spread between MFMAs; nz / sc / w4:
-  // the fragment's constants, set by its pair-0 call.
+  // * scale), bit-identical to the dequant kernel for zero-points that are whole
+  // numbers from 0 to 1024, which is what checkpoints hold (q - zp is a difference
+  // of fp16 numbers).  One pair at a time, so that the arithmetic can be spread
+  // between MFMAs; nz / sc / w4: the fragment's constants, set by its pair-0 call.
   __device__ __forceinline__ uint32_t dqp(const Raw& r, int f, int j, int k, h2_t& nz, h2_t& sc,
                                           uint32_t& w4) const {
     if constexpr (WBITS == 16) {
@@ -395,6 +399,43 @@ struct TileSeg {
       return as_u32((as_h2(pr) + nz) * sc);
     }
   }
+  // The same for any zero-point, as the dequant kernel computes it.
+  __device__ __forceinline__ h8_t dqx(const Raw& r, int f, int j) const {
+    const float scale = h2f((uint16_t)(r.s2[f][j] & 0xFFFFu)), zp = h2f((uint16_t)(r.s2[f][j] >> 16));
+    u4_t o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      uint32_t q[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        q[e] = WBITS == 4 ? (r.w[f][j][0] >> (8 * k + 4 * e)) & 0xFu
+                          : (r.w[f][j][k >> 1] >> (16 * (k & 1) + 8 * e)) & 0xFFu;
+      const float lo = ((float)q[0] - zp) * scale, hi = ((float)q[1] - zp) * scale;
+      o[k] = (uint32_t)f2h(lo) | ((uint32_t)f2h(hi) << 16);
+    }
+    return __builtin_bit_cast(h8_t, o);
+  }
+
+  // Zero-points that dqp rounds, in the (scale, zero) words that a lane looks at
+  // in a step (lane group g: weight row + 4 (g / J), MFMA k-step g % J): the OR of
+  // their fractions and their maximum, as patterns (1024 is 0x6400, a negative
+  // number is larger; a NaN is one either way).
+  struct Zp {
+    uint32_t frac = 0, top = 0;
+    __device__ __forceinline__ void look(uint32_t w) {
+      typedef uint16_t us2_t __attribute__((ext_vector_type(2)));
+      const _Float16 z = __builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+      frac |= __builtin_bit_cast(uint16_t, (_Float16)__builtin_amdgcn_fracth(z));
+      top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2_t, top),
+                                                                   __builtin_bit_cast(us2_t, w)));
+    }
+    __device__ __forceinline__ bool found() const { return frac != 0 || (top >> 16) > 0x6400u; }
+  };
+  __device__ __forceinline__ uint32_t zp_word(const lds8* st) const {
+    static_assert(!kAnyZp || NF * T::J == 4, "a wave looks at every word of its rows");
+    return lds_ld<uint32_t>(st + os + T::SW * 16 * (g / T::J) + 4 * (g % T::J));
+  }
+
   __device__ __forceinline__ h8_t dq(const Raw& r, int f, int j) const {
     u4_t o;
     h2_t nz, sc;
@@ -409,6 +450,10 @@ struct TileSeg {
     return lds_ld<h8_t>(st + ox[q / MT] + 16 * (q % MT) * T::XRow);
   }
 
+  __device__ __forceinline__ lds8* next(lds8* st) const {  // the ring's stage after st
+    return st + T::kStage == ring + T::D * T::kStage ? ring : st + T::kStage;
+  }
+
   // the segment's first copies
   __device__ __forceinline__ void start() const {
 #pragma unroll
@@ -416,10 +461,65 @@ struct TileSeg {
   }
 
   // the segment's K loop, after start(); stores issued since then only make
-  // the first wait stricter (copies retire in order among themselves)
+  // the first wait stricter (copies retire in order among themselves).
+  // kAnyZp: a tile with zero-points that dqp rounds is computed again, with dqx:
+  // 96 x 7168 x 5120 INT4 21 us, with such zero-points 51.  The look costs 96 x 7168 x
+  // 5120 20.7 -> 21.3, 64 x 5120 x 17408 52.8 -> 56.4, 128 x 34816 x 5120 79.5 -> 81.3;
+  // a branch in every step took the first two to 25.2 and 62.8, a fifth wave that
+  // looks all three to 23.1, 57.1 and 98.6.
   __device__ __forceinline__ void run(f4_t (&acc)[NF][MT], int t) const {
+    Zp zp;
+    loop(acc, t, zp);
+    if constexpr (kAnyZp) {
+      // the waves' findings, in the one stage that start() does not fill
+      typedef __attribute__((address_space(3))) uint32_t lds_u1;
+      lds8* const found = ring + (T::D - 1) * T::kStage;
+      *(lds_u1*)(found + 4 * wave) = __any(zp.found());
+      ring_barrier();
+      const u4_t f = lds_ld<u4_t>(found);
+      if (__builtin_amdgcn_readfirstlane(f[0] | f[1] | f[2] | f[3])) {
+        start();
+        loop_any_zp(acc, t);
+      }
+    }
+  }
+  __device__ __forceinline__ void loop_any_zp(f4_t (&acc)[NF][MT], int t) const {
+    const bool tail = ka + nk * T::KS > ke;
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[f][m] = f4_t{0.f, 0.f, 0.f, 0.f};
+    lds8 *cur = ring, *far = ring + (T::D - 1) * T::kStage;
+    for (int i = 0; i < nk; ++i) {
+      Raw raw;
+      wait_copies<(T::D - 2) * T::kPer>();
+      ring_barrier();
+      if (tail && i + 1 == nk) clear_tail(nk - 1, cur, t);
+      issue(i + T::D - 1, far);
+      load_raw(cur, raw);
+#pragma unroll
+      for (int j = 0; j < T::J; ++j) {
+        h8_t b[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) b[f] = dqx(raw, f, j);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const h8_t a = xfrag(cur, j * MT + m);
+#pragma unroll
+          for (int f = 0; f < NF; ++f)
+            acc[f][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[f], a, acc[f][m], 0, 0, 0);
+        }
+      }
+      far = cur;
+      cur = next(cur);
+    }
+    wait_copies<0>();
+    ring_barrier();
+  }
+  __device__ __forceinline__ void loop(f4_t (&acc)[NF][MT], int t, Zp& zp) const {
     const bool tail = ka + nk * T::KS > ke;
     Raw raw;
+    uint32_t zw = 0;
     h8_t a[T::P], b[NF];
     lds8 *cur = ring, *far = ring + (T::D - 1) * T::kStage;
     for (int i = 0; i < nk; ++i) {
@@ -429,6 +529,10 @@ struct TileSeg {
       load_raw(cur, raw);
 #pragma unroll
       for (int q = 0; q < T::P; ++q) a[q] = xfrag(cur, q);
+      if constexpr (kAnyZp) {  // (at the word of the step before: it is there)
+        zp.look(zw);
+        zw = zp_word(cur);
+      }
 #pragma unroll
       for (int f = 0; f < NF; ++f) b[f] = dq(raw, f, 0);
       const Src sc0 = src(i + T::D - 1, far);
@@ -458,8 +562,9 @@ struct TileSeg {
         for (int f = 0; f < NF; ++f) if (j + 1 < T::J) b[f] = __builtin_bit_cast(h8_t, bn[f]);
       }
       far = cur;
-      cur = cur + T::kStage == ring + T::D * T::kStage ? ring : cur + T::kStage;
+      cur = next(cur);
     }
+    if constexpr (kAnyZp) zp.look(zw);
     wait_copies<0>();  // no copy may land once the ring is reused
     ring_barrier();
   }

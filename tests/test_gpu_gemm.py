@@ -415,3 +415,33 @@ def test_tile_gemm_one_hot_and_infinite_rows(dev, bits, M, N, K):
             assert np.array_equal(y[r], W[:, k]), (r, k)
     nz = W[:, K - 1] != 0
     assert np.array_equal(y[2][nz], np.where(W[nz, K - 1] > 0, np.inf, -np.inf).astype(np.float16))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K", [(17, 70, 1056), (48, 8259, 352), (64, 8259, 1184), (64, 16500, 608),
+                                   (96, 16500, 736), (128, 16500, 352), (255, 300, 2080)])
+def test_tile_gemm_zero_points_of_any_value(dev, bits, M, N, K):
+    """fp16((q - zp) * scale) holds for every zero-point below 256 rows, whole
+    number or not, in every tile shape (32 x 64 .. 128 x 128 in this order):
+    row r of x = e_k(r) gives column k(r) of the oracle's dequantised weight bit
+    for bit where blocks with other zero-points sit among the usual ones, in
+    some weight rows only, and in a last partial step."""
+    g = S.gen(3 * M + N + K + bits)
+    w, sz = S.weight(N, K, bits, g)
+    z = sz.view(N, K // 32, 2)[:, :, 1]
+    odd = torch.tensor([0.5, 7.25, -0.5, -100.0625, 1e-6, 0.1, 1024.0, 1025.0, 2047.0, 3001.0,
+                        -1000.5, 60000.0]).half()
+    pick = torch.randint(0, len(odd), z.shape, generator=g)
+    where = torch.rand(z.shape, generator=g) < 0.02
+    where[: N // 3, : K // 64] = False  # steps without any
+    where[:, -1] |= torch.rand(N, generator=g) < 0.3
+    z[where] = odd[pick[where]]
+    W = O.dequant(w.numpy(), sz.numpy(), bits)
+    assert np.all(np.isfinite(W))
+    ks = [(r * 97 + r // 3) % K for r in range(M)]
+    ks[1] = K - 1
+    x = torch.zeros(M, K, dtype=torch.float16)
+    x[torch.arange(M), torch.tensor(ks)] = 1.0
+    y = int4_hip.dbg_gemm(x.to(dev), w.to(dev), sz.to(dev), M, N, K).cpu().numpy()
+    for r, k in enumerate(ks):
+        assert np.array_equal(y[r], W[:, k]), (r, k)
