@@ -127,6 +127,20 @@ def test_gemm_workspace_sizes():
         ws(8, 5120, 100, 4)                           # K % 32 != 0
 
 
+@pytest.mark.parametrize("bits,step", [(4, 64), (8, 64), (16, 64)])
+def test_gemm_shares_k_in_whole_steps(bits, step):
+    """M >= 256: what workgroups share of a tile is a whole number of the
+    kernel's K steps.  One tile of one step cannot be shared (no workspace),
+    one of many steps is."""
+    def ws(K):
+        b = C.c_size_t(123)
+        R.call("r4q_gemm_workspace_bytes", 256, 256, K, bits, C.byref(b))
+        return b.value
+    assert ws(step // 2) == 0 and ws(step) == 0
+    assert ws(step + 32) == (0 if bits < 16 else 2 * 256 * 256 * 2)
+    assert ws(16 * step) > 0
+
+
 def test_gate_up_silu_split_point():
     """Whole 64-row units in multiples of 256 (the CU count), the rest as
     fp32 pairs; fewer than 256 units: all units."""
