@@ -675,20 +675,22 @@ __global__ __launch_bounds__(256 * MG, 2) void gemm_tile_kernel(
         }
       }
     } else {
-      // fp16 partials in the order of the outputs a row at a time: element
-      // ((wc MTT + M-block) 16 + col) 4 + g, then the lane's 4 NF outputs
+      // fp16 partials in 16-byte pieces, outputs 8 h .. 8 h + 7 of the lane's 4 NF
+      // at piece ((wc MTT + M-block) NF / 2 + h) 64 + lane: a store instruction
+      // of a wave covers whole lines
       if constexpr (MG == 2) {
         const int tl = ctile - dp, j = w - sk_owner((int64_t)tl * U, TU, sk);
-        uint16_t* pt = part + ((int64_t)tl * maxseg + j) * (T::BM * T::BN);
+        u4_t* pt = reinterpret_cast<u4_t*>(part + ((int64_t)tl * maxseg + j) * (T::BM * T::BN));
+        pt += (wc * MT * MG + MT * sg.mg) * (NF / 2 * 64) + 16 * sg.g + sg.col;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-          uint16_t* p = pt + (((wc * MT * MG + MT * sg.mg + m) * 16 + sg.col) * 4 + sg.g) * (4 * NF);
 #pragma unroll
-          for (int f = 0; f < NF; f += 2)
-            *reinterpret_cast<u4_t*>(p + 4 * f) =
-                u4_t{cvt_pk_h(acc[f][m][0], acc[f][m][1]), cvt_pk_h(acc[f][m][2], acc[f][m][3]),
-                     cvt_pk_h(acc[f + 1][m][0], acc[f + 1][m][1]),
-                     cvt_pk_h(acc[f + 1][m][2], acc[f + 1][m][3])};
+          for (int h = 0; h < NF / 2; ++h)
+            pt[(m * (NF / 2) + h) * 64] = u4_t{
+                cvt_pk_h(acc[2 * h][m][0], acc[2 * h][m][1]),
+                cvt_pk_h(acc[2 * h][m][2], acc[2 * h][m][3]),
+                cvt_pk_h(acc[2 * h + 1][m][0], acc[2 * h + 1][m][1]),
+                cvt_pk_h(acc[2 * h + 1][m][2], acc[2 * h + 1][m][3])};
         }
       }
     }
@@ -696,28 +698,36 @@ __global__ __launch_bounds__(256 * MG, 2) void gemm_tile_kernel(
 }
 
 // Y = fp16(sum of the segments of each shared tile, in segment order, in
-// fp32).  A thread takes 16 bytes of every segment, consecutive threads
-// consecutive bytes, and writes that many outputs of one row.
+// fp32).  A thread takes a 16-byte piece of every segment and writes that many
+// outputs of one row; 2 NF consecutive threads a row of a wave's 16 NF outputs.
+// Blocks are placed as the GEMM's are, so that a tile is summed on the XCD that
+// wrote its segments.  Read on any XCD, the partials of a following GEMM into the
+// same workspace took up to 14 us to be accepted (its kernel's own clock; the less
+// it had read before them, the longer), it seems for the copies that the other L2s
+// held: 1024 x 4096 x 1024 INT4 36 us, with whole lines per store 35, with the
+// placement 27; 512 x 1024 x 1024 INT8 21, 19 and 14; 512 x 17408 x 5120 INT4 108, 107.
 template <class T>
 __global__ __launch_bounds__(256) void gemm_tile_reduce_kernel(const uint16_t* __restrict__ part,
                                                                uint16_t* __restrict__ Y, int M,
                                                                int N, int dp, int sk, int U,
                                                                int maxseg, int vec) {
   constexpr int NF = T::BN / 64, MTT = T::BM / 16, E = T::kOut, kPerTile = T::BM * T::BN / E;
-  const int64_t gt = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t gt = (int64_t)xcd_order(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   const int ntm = (M + T::BM - 1) / T::BM, ntn = (N + T::BN - 1) / T::BN;
-  const int tl = (int)(gt / kPerTile), e = (int)(gt % kPerTile) * E;
+  const int tl = (int)(gt / kPerTile), x = (int)(gt % kPerTile);
   if (tl >= ntm * ntn - dp) return;
   const int64_t TU = (int64_t)(ntm * ntn - dp) * U;
   const int w0 = sk_owner((int64_t)tl * U, TU, sk), w1 = sk_owner((int64_t)tl * U + U - 1, TU, sk);
   const int nseg = w1 - w0 + 1;
   if (nseg == 1) return;  // computed whole: written by the GEMM
   const int tile = dp + tl;
-  const int r = e / (16 * NF);  // (wc MTT + M-block) 16 + col
-  const int row = (tile / ntn) * T::BM + r % (16 * MTT);
-  const int n = (tile % ntn) * T::BN + 16 * NF * (r / (16 * MTT)) + e % (16 * NF);
+  constexpr int G = 2 * NF;  // threads of a row of a wave's 16 NF outputs
+  const int q = x % G, col = x / G % 16, wm = x / (16 * G);  // wm = wc MTT + M-block
+  const int row = (tile / ntn) * T::BM + 16 * (wm % MTT) + col;
+  const int n = (tile % ntn) * T::BN + 16 * NF * (wm / MTT) + E * q;
   if (row >= M || n >= N) return;
-  const u4_t* p = reinterpret_cast<const u4_t*>(part + (int64_t)tl * maxseg * (T::BM * T::BN) + e);
+  const u4_t* p = reinterpret_cast<const u4_t*>(part + (int64_t)tl * maxseg * (T::BM * T::BN)) +
+                  (wm * (NF / 2) + q % (NF / 2)) * 64 + 16 * (q / (NF / 2)) + col;
   float v[E];
   auto add = [&](u4_t x, bool first) {
 #pragma unroll
