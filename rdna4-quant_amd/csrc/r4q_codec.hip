@@ -80,20 +80,27 @@ __device__ __forceinline__ uint32_t fp8_encode_pair(uint32_t h) {
   return __builtin_bit_cast(uint32_t, c) | __builtin_bit_cast(uint32_t, sign);
 }
 
+// Turns of the FP8 codecs.  Up to kOneTurn elements one turn each: that many
+// workgroups fit the chip at once, and the time is that of a thread's own work
+// (encode, one turn / four: 64 K values 2.3 / 2.9 us, 1 M 2.5 / 3.0, 8.4 M 5.8 / 6.1, 33.5 M
+// 20.0 / 18.9; decode on 8 codes 2.2 / 2.7, 2.5 / 2.9, 5.1 / 5.5, 16.2 / 15.7).
+constexpr int64_t kOneTurn = (int64_t)1 << 23;
+
 // Four elements per thread and turn.  The scalar recipe's ~22 instructions per
 // element were as long as the stream: 33.5 M values 27 -> 19.5 us (5.2 TB/s).
 // Eight elements (16-byte loads where src is so aligned) measured the same.
+template <int TURNS>
 __global__ __launch_bounds__(256) void fp16_to_fp8_kernel(const uint16_t* __restrict__ src,
                                                           uint8_t* __restrict__ dst, int64_t n) {
-  const int64_t p0 = (int64_t)blockIdx.x * (256 * kTurns) + threadIdx.x, np = n / 4;
-  u2_t v[kTurns];
+  const int64_t p0 = (int64_t)blockIdx.x * (256 * TURNS) + threadIdx.x, np = n / 4;
+  u2_t v[TURNS];
 #pragma unroll
-  for (int i = 0; i < kTurns; ++i) {
+  for (int i = 0; i < TURNS; ++i) {
     const int64_t p = p0 + 256 * i;
     if (p < np) v[i] = reinterpret_cast<const u2_t*>(src)[p];
   }
 #pragma unroll
-  for (int i = 0; i < kTurns; ++i) {
+  for (int i = 0; i < TURNS; ++i) {
     const int64_t p = p0 + 256 * i;
     if (p < np)  // bytes 0 and 2 of the two pairs
       reinterpret_cast<uint32_t*>(dst)[p] = __builtin_amdgcn_perm(
@@ -104,23 +111,24 @@ __global__ __launch_bounds__(256) void fp16_to_fp8_kernel(const uint16_t* __rest
 }
 
 // VEC = 8 codes per thread and turn where src is 8-byte and dst 16-byte
-// aligned, else 1.  33.5 M codes: 16 us (6.3 TB/s) with 8, 26 with 1; 41 with 1
+// aligned, else 1 (four turns at every size: one was as fast up to 512 K codes and
+// slower from 1 M on).  33.5 M codes: 16 us (6.3 TB/s) with 8, 25 with 1; 40 with 1
 // code per thread in all.
-template <int VEC>
+template <int VEC, int TURNS>
 __global__ __launch_bounds__(256) void fp8_to_fp16_kernel(const uint8_t* __restrict__ src,
                                                           uint16_t* __restrict__ dst, int64_t n) {
   const h2_t k256 = as_h2(0x5C005C00u);  // (256, 256): exact, subnormals included
-  const int64_t p0 = (int64_t)blockIdx.x * (256 * kTurns) + threadIdx.x, np = n / VEC;
-  u2_t c[kTurns];
+  const int64_t p0 = (int64_t)blockIdx.x * (256 * TURNS) + threadIdx.x, np = n / VEC;
+  u2_t c[TURNS];
 #pragma unroll
-  for (int i = 0; i < kTurns; ++i) {
+  for (int i = 0; i < TURNS; ++i) {
     const int64_t p = p0 + 256 * i;
     if (p >= np) continue;
     if constexpr (VEC == 8) c[i] = reinterpret_cast<const u2_t*>(src)[p];
     else c[i][0] = src[p];
   }
 #pragma unroll
-  for (int i = 0; i < kTurns; ++i) {
+  for (int i = 0; i < TURNS; ++i) {
     const int64_t p = p0 + 256 * i;
     if (p >= np) continue;
     u4_t o;
@@ -139,8 +147,8 @@ __global__ __launch_bounds__(256) void fp8_to_fp16_kernel(const uint8_t* __restr
 }
 
 // workgroups for n pieces of work; at least one (it also does the remainder)
-unsigned turn_grid(int64_t n) {
-  return (unsigned)std::max<int64_t>(1, (n + 256 * kTurns - 1) / (256 * kTurns));
+unsigned turn_grid(int64_t n, int turns = kTurns) {
+  return (unsigned)std::max<int64_t>(1, (n + 256 * turns - 1) / (256 * turns));
 }
 
 bool aligned(const void* p, int a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
@@ -178,9 +186,15 @@ extern "C" int r4q_fp16_to_fp8(const void* src, void* dst, int64_t n, void* stre
   if (n == 0) return R4Q_OK;
   R4Q_REQUIRE(src && dst, "fp16_to_fp8: null pointer");
   R4Q_REQUIRE(r4q::aligned(src, 8) && r4q::aligned(dst, 4), "fp16_to_fp8: misaligned pointer");
-  hipLaunchKernelGGL(r4q::fp16_to_fp8_kernel, dim3(r4q::turn_grid(n / 4)), dim3(256), 0,
-                     r4q::as_stream(stream), static_cast<const uint16_t*>(src),
-                     static_cast<uint8_t*>(dst), n);
+  const auto* sp = static_cast<const uint16_t*>(src);
+  auto* dp = static_cast<uint8_t*>(dst);
+  const hipStream_t st = r4q::as_stream(stream);
+  if (n <= r4q::kOneTurn)
+    hipLaunchKernelGGL(r4q::fp16_to_fp8_kernel<1>, dim3(r4q::turn_grid(n / 4, 1)), dim3(256), 0, st,
+                       sp, dp, n);
+  else
+    hipLaunchKernelGGL(r4q::fp16_to_fp8_kernel<r4q::kTurns>, dim3(r4q::turn_grid(n / 4)), dim3(256),
+                       0, st, sp, dp, n);
   return r4q::launch_status("fp16_to_fp8");
 }
 
@@ -191,11 +205,14 @@ extern "C" int r4q_fp8_to_fp16(const void* src, void* dst, int64_t n, void* stre
   const auto* sp = static_cast<const uint8_t*>(src);
   auto* dp = static_cast<uint16_t*>(dst);
   const hipStream_t st = r4q::as_stream(stream);
-  if (r4q::aligned(src, 8) && r4q::aligned(dst, 16))
-    hipLaunchKernelGGL(r4q::fp8_to_fp16_kernel<8>, dim3(r4q::turn_grid(n / 8)), dim3(256), 0, st, sp,
-                       dp, n);
+  if (!r4q::aligned(src, 8) || !r4q::aligned(dst, 16))
+    hipLaunchKernelGGL((r4q::fp8_to_fp16_kernel<1, r4q::kTurns>), dim3(r4q::turn_grid(n)), dim3(256),
+                       0, st, sp, dp, n);
+  else if (n <= r4q::kOneTurn)
+    hipLaunchKernelGGL((r4q::fp8_to_fp16_kernel<8, 1>), dim3(r4q::turn_grid(n / 8, 1)), dim3(256), 0,
+                       st, sp, dp, n);
   else
-    hipLaunchKernelGGL(r4q::fp8_to_fp16_kernel<1>, dim3(r4q::turn_grid(n)), dim3(256), 0, st, sp, dp,
-                       n);
+    hipLaunchKernelGGL((r4q::fp8_to_fp16_kernel<8, r4q::kTurns>), dim3(r4q::turn_grid(n / 8)),
+                       dim3(256), 0, st, sp, dp, n);
   return r4q::launch_status("fp8_to_fp16");
 }

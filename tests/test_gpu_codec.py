@@ -86,6 +86,21 @@ def test_fp8_codecs_at_every_alignment(dev, n):
         assert np.array_equal(got[ok], want[ok])
 
 
+@pytest.mark.parametrize("n", [(1 << 23) - 1, 1 << 23, (1 << 23) + 1, (1 << 23) + 8200])
+def test_fp8_codecs_either_side_of_one_turn(dev, n):
+    """The last size with one turn per thread and the first with four, with
+    partial turns and remainders: every code against the tables."""
+    bits = torch.arange(n, dtype=torch.int32, device=dev) * 40503 + n
+    x = bits.to(torch.int16).view(torch.float16)
+    enc = torch.from_numpy(fp8_golden_table()).to(dev)
+    assert torch.equal(int4_hip.fp16_to_fp8(x), enc[(bits & 0xFFFF).long()])
+    codes = (bits >> 3).to(torch.uint8)
+    val = torch.from_numpy(O.fp8_value(np.arange(256, dtype=np.uint8))).to(dev)
+    want = val[codes.long()]
+    got = int4_hip.fp8_to_fp16(codes).double()
+    assert torch.equal(got[~want.isnan()], want[~want.isnan()])
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("N,K", [(1, 32), (1, 8160), (1, 8192), (255, 32), (257, 64), (3, 8224)])
 def test_dequant_turn_edges(dev, bits, N, K):
