@@ -88,32 +88,9 @@ __device__ __forceinline__ h8_t skinny_b(const u4_t w, uint32_t s2, int d) {
   }
 }
 
-// LDS-qualified byte pointer: ring addresses stay 32-bit LDS offsets (a
-// generic pointer into LDS is a 64-bit value the compiler keeps in VGPRs).
-typedef __attribute__((address_space(3))) uint8_t lds8;
 template <class T>
 __device__ __forceinline__ T lds_ld(const lds8* p) {
   return *(const __attribute__((address_space(3))) T*)p;
-}
-__device__ __forceinline__ uint32_t lds_off(const lds8* p) {
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p);
-}
-
-// Global -> LDS copy of 16 (4) bytes per lane: lane l's bytes land at
-// lds + 16 l (4 l); a uniform 64-bit base in SGPRs and a 32-bit byte offset
-// per lane.  Written as inline assembly so that the compiler's wait-count
-// tracking does not see the copies: it would otherwise wait for every copy in
-// flight before any LDS read of the ring; the kernels count and wait for their
-// own copies (wait_copies) instead.
-__device__ __forceinline__ void copy16s(const void* base, uint32_t off, lds8* lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_off(lds)),
-               "v"(off), "s"(base)
-               : "memory");
-}
-__device__ __forceinline__ void copy4s(const void* base, uint32_t off, lds8* lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_off(lds)),
-               "v"(off), "s"(base)
-               : "memory");
 }
 
 template <int N>

@@ -62,18 +62,7 @@ __global__ __launch_bounds__(256) void embed_gather_kernel(const int64_t* __rest
 constexpr int kFaRows = 64;        // query rows of a workgroup
 constexpr int kFaTile = 32 * 256;  // bytes of a block's K (or V) in LDS: K, K, V, V
 
-typedef __attribute__((address_space(3))) uint8_t lds8;
 typedef short s4_t __attribute__((ext_vector_type(4)));
-
-// Global -> LDS copy of 16 bytes per lane (lane l's land at lds + 16 l), as inline
-// assembly so that the compiler does not wait for it before unrelated LDS reads:
-// the kernel waits for its own copies.
-__device__ __forceinline__ void copy16(const void* src, lds8* lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(
-                   __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds)),
-               "v"(src)
-               : "memory");
-}
 
 // maximum over the lanes n, n + 16, n + 32, n + 48, in all of them
 __device__ __forceinline__ float max_groups(float v) {
