@@ -396,7 +396,7 @@ R4Q_API int r4q_decode_profile(r4q_ctx* ctx, const r4q_model* m, const void* hid
  * "split_reduce" (1 = batched decode steps reduce the split-K partials of
  * the qkv, o and down projections in their own launches, not in the
  * attention prologue / row norm that consume them), "gemm_kernel" (1 or 2,
- * without effect: one kernel serves every M > 16), "gemv_skew"
+ * accepted, neither kept nor of any effect: one kernel serves every M > 16), "gemv_skew"
  * (GEMV on an even grid of more than 256 equal shares: the first half of the
  * workgroups takes value - 1 steps more and the second half value - 1 fewer;
  * 1 = equal shares; default 2 on a 512-workgroup grid of at least 4 steps

@@ -30,7 +30,7 @@ int launch_status(const char* what);
 //   attn_splits   R4Q_ATTN_SPLITS   flash-decode splits: 1 .. 128
 //   skinny_splits R4Q_SKINNY_SPLITS skinny-GEMM K splits: 1 .. 8
 //   gemm_splits   R4Q_GEMM_SPLITS   tile GEMM: 1 whole tiles, 2 .. 16 stream-K workgroups per tile
-//   gemm_kernel   R4Q_GEMM_KERNEL   1 or 2, without effect: one kernel serves every M > 16
+//   gemm_kernel   R4Q_GEMM_KERNEL   1 or 2, accepted and dropped: one kernel serves every M > 16
 //   gemv_skew     R4Q_GEMV_SKEW     GEMV on an even grid of more than 256 equal shares: the
 //                                   first half takes value - 1 steps more, the second half
 //                                   value - 1 fewer (1 = equal shares)
@@ -40,7 +40,7 @@ int launch_status(const char* what);
 struct Tuning {
   std::atomic<int> gemv_lpr{0}, gemv_wgs{0}, gemv_ub{0};
   std::atomic<int> attn_splits{0}, skinny_splits{0}, gemm_splits{0};
-  std::atomic<int> split_reduce{0}, gemm_kernel{0}, gemv_skew{0};
+  std::atomic<int> split_reduce{0}, gemv_skew{0};
 };
 Tuning& tuning();
 

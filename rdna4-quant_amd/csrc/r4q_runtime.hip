@@ -34,7 +34,7 @@ namespace {
 struct Knob {
   const char* name;  // r4q_tune name; the environment variable is R4Q_<NAME>
   const char* env;
-  std::atomic<int> Tuning::*field;
+  std::atomic<int> Tuning::*field;  // nullptr: accepted, without effect
   int lo, hi;
   bool pow2;
 };
@@ -46,7 +46,7 @@ const Knob kKnobs[] = {
     {"skinny_splits", "R4Q_SKINNY_SPLITS", &Tuning::skinny_splits, 1, 8, false},
     {"gemm_splits", "R4Q_GEMM_SPLITS", &Tuning::gemm_splits, 1, 16, false},
     {"split_reduce", "R4Q_SPLIT_REDUCE", &Tuning::split_reduce, 1, 1, false},
-    {"gemm_kernel", "R4Q_GEMM_KERNEL", &Tuning::gemm_kernel, 1, 2, false},
+    {"gemm_kernel", "R4Q_GEMM_KERNEL", nullptr, 1, 2, false},
     {"gemv_skew", "R4Q_GEMV_SKEW", &Tuning::gemv_skew, 1, 8, false},
 };
 
@@ -68,7 +68,8 @@ int env_knob(const Knob& k) {
 Tuning& tuning() {
   static Tuning t;
   static const bool init = [] {
-    for (const Knob& k : kKnobs) (t.*k.field).store(env_knob(k));
+    for (const Knob& k : kKnobs)
+      if (k.field) (t.*k.field).store(env_knob(k));
     return true;
   }();
   (void)init;
@@ -112,7 +113,7 @@ extern "C" int r4q_tune(const char* name, int value) {
     if (strcmp(name, k.name) != 0) continue;
     R4Q_REQUIRE(value == 0 || r4q::knob_ok(k, value), "tune: %s=%d outside [%d, %d]%s", name,
                 value, k.lo, k.hi, k.pow2 ? " (power of two)" : "");
-    (r4q::tuning().*k.field).store(value);
+    if (k.field) (r4q::tuning().*k.field).store(value);
     return R4Q_OK;
   }
   return r4q::fail(R4Q_EINVAL, "tune: unknown knob '%s'", name);
