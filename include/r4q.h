@@ -127,6 +127,12 @@ R4Q_API int r4q_gemm(const void* x, const void* w, const void* sz, void* y,
  * dequant_matmul_out (hip:1973-1988). */
 R4Q_API int r4q_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int wbits,
                                      size_t* bytes);
+/* How r4q_gemm_ws with ws_bytes of workspace computes M > 16 rows, without
+ * running it (no counterpart in the reference; for tests and measurement):
+ * out[0], out[1] = rows and columns of an output tile, out[2] = tiles computed
+ * whole, out[3] = workgroups sharing the K units of the others.  n >= 4. */
+R4Q_API int r4q_gemm_plan(int64_t M, int64_t N, int64_t K, int wbits, size_t ws_bytes,
+                          int32_t* out, int64_t n);
 /* r4q_gemm with a caller-owned workspace of ws_bytes (NULL / 0: no split). */
 R4Q_API int r4q_gemm_ws(const void* x, const void* w, const void* sz, void* y,
                         int64_t M, int64_t N, int64_t K, int wbits, void* ws,

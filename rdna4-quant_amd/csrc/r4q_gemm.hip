@@ -1479,6 +1479,15 @@ TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int wbits, size_t ws_bytes) 
   return pl;
 }
 
+void gemm_plan(int64_t M, int64_t N, int64_t K, int wbits, size_t ws_bytes, int32_t* out) {
+  const TileShape s = tile_shape(M, N, K, wbits);
+  const TilePlan pl = tile_plan(M, N, K, wbits, ws_bytes);
+  out[0] = 16 * s.mt * s.mg;
+  out[1] = 64 * s.nf;
+  out[2] = pl.dp;
+  out[3] = pl.sk;
+}
+
 size_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int wbits) {
   return tile_plan(M, N, K, wbits, (size_t)-1).ws;
 }

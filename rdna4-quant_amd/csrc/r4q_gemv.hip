@@ -994,6 +994,16 @@ extern "C" int r4q_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int wbi
   return R4Q_OK;
 }
 
+extern "C" int r4q_gemm_plan(int64_t M, int64_t N, int64_t K, int wbits, size_t ws_bytes,
+                             int32_t* out, int64_t n) {
+  R4Q_REQUIRE(out && n >= 4, "gemm_plan: need room for 4 values");
+  R4Q_REQUIRE(M > r4q::kSkinnyMaxRows && N >= 1 && K >= 32 && K % 32 == 0 &&
+                  (wbits == 4 || wbits == 8 || wbits == 16),
+              "gemm_plan: bad shape or format (M > 16)");
+  r4q::gemm_plan(M, N, K, wbits, ws_bytes, out);
+  return R4Q_OK;
+}
+
 extern "C" int r4q_gemm_ws(const void* x, const void* w, const void* sz, void* y, int64_t M,
                            int64_t N, int64_t K, int wbits, void* ws, size_t ws_bytes,
                            void* stream) {

@@ -47,6 +47,8 @@ constexpr int64_t kSkinnyMaxRows = 16;
 // launch.
 // Workspace bytes for the best split count of a shape (0: none needed).
 size_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int wbits);
+// out[4]: tile rows, tile columns, whole tiles, stream-K workgroups (M > 16).
+void gemm_plan(int64_t M, int64_t N, int64_t K, int wbits, size_t ws_bytes, int32_t* out);
 int gemm_mfma_launch(const void* x, const void* w, const void* sz, void* y, int64_t M, int64_t N,
                      int64_t K, int wbits, hipStream_t st, void* ws = nullptr,
                      size_t ws_bytes = 0);

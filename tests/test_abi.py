@@ -141,6 +141,29 @@ def test_gemm_shares_k_in_whole_steps(bits, step):
     assert ws(16 * step) > 0
 
 
+def test_gemm_plan_tiles():
+    """M > 16: the tile by the work of the most loaded of 256 CUs below 256 rows,
+    256 x 256 from there on, split with a workspace only; operands of 4 GiB and
+    more in whole tiles of at most 128 rows; one to 16 rows are refused."""
+    def plan(M, N, K, bits, ws=1 << 40):
+        v = (C.c_int32 * 4)()
+        R.call("r4q_gemm_plan", M, N, K, bits, ws, v, 4)
+        return tuple(v)
+    assert plan(17, 7168, 5120, 4) == (32, 64, 112, 0)
+    assert plan(96, 7168, 5120, 4) == (48, 64, 224, 0)
+    assert plan(96, 7168, 5120, 16) == (64, 64, 224, 0)  # no 48 x 64 for FP16
+    assert plan(96, 34816, 5120, 8) == (96, 128, 272, 0)
+    assert plan(200, 34816, 5120, 4) == (128, 128, 544, 0)
+    assert plan(512, 17408, 5120, 4) == (256, 256, 0, 256)
+    assert plan(512, 17408, 5120, 4, 0) == (256, 256, 136, 0)
+    assert plan(512, 34816, 5120, 4) == (256, 256, 256, 256)
+    assert plan(512, 151936, 5120, 16) == (256, 256, 1188, 0)
+    assert plan(512, 151936, 16384, 16)[0] <= 128 and plan(512, 151936, 16384, 16)[3] == 0
+    for bad in ((16, 64, 64, 4), (17, 64, 33, 4), (17, 64, 64, 5)):
+        with pytest.raises(RuntimeError):
+            plan(*bad)
+
+
 def test_gate_up_silu_split_point():
     """Whole 64-row units in multiples of 256 (the CU count), the rest as
     fp32 pairs; fewer than 256 units: all units."""

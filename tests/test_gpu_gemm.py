@@ -96,8 +96,8 @@ def test_skinny_gemm_one_hot_columns_exact(dev, bits):
 @pytest.mark.parametrize("M,N,K", [(300, 1000, 2048), (257, 520, 32), (600, 256, 4096),
                                    (512, 7168, 5120), (256, 255, 96)])
 def test_ring_gemm_ragged_and_split(dev, bits, M, N, K):
-    """M >= 256: the 256 x 256 LDS-ring kernel, with ragged M / N tiles,
-    K loops shorter than the copy ring (K = 32, 96), and split-K over a
+    """M >= 256: 256 x 256 tiles, ragged in M and N, K loops shorter than the
+    copy ring (K = 32, 96), and split-K over a
     workspace (few tiles, long K)."""
     got, want = _run(dev, bits, M, N, K, seed=M + 3 * N + K + bits)
     assert np.all(np.isfinite(got))
@@ -111,7 +111,7 @@ def test_ring_gemm_ragged_and_split(dev, bits, M, N, K):
 def test_ring_gemm_one_hot_columns_exact(dev, bits, N, K):
     """Row r of x = e_k(r) over 300 rows: y[r] is column k(r) of the
     dequantised weight, bit for bit -- in one pass and with the K loop split
-    (fp32 partials of zeros and one exact product)."""
+    (fp16 partials of zeros and one exact product)."""
     g = S.gen(43 + bits + K)
     M = 300
     w, sz = S.weight(N, K, bits, g)
@@ -127,7 +127,8 @@ def test_ring_gemm_one_hot_columns_exact(dev, bits, N, K):
 
 
 def test_ring_gemm_split_matches_unsplit(dev):
-    """The split-K result equals the one-pass result within fp32 rounding."""
+    """The split-K result equals the one-pass result within the rounding of
+    its fp16 partials."""
     import ctypes as C
     import r4q_lib as R
     g = S.gen(77)
@@ -239,7 +240,7 @@ def _ref32(x, w, sz, bits):
 def test_ring_gemm_whole_tile_rounds_then_stream_k(dev, bits):
     """576 tiles of 256 x 256 (more than two rounds of 256 workgroups): the
     first two rounds' 512 tiles are computed whole, the remaining 64 tiles'
-    K units are shared by 256 stream-K workgroups (pieces of tiles as fp32
+    K units are shared by 256 stream-K workgroups (pieces of tiles as fp16
     partials, summed in segment order)."""
     import ctypes as C
     import r4q_lib as R
@@ -262,8 +263,8 @@ def test_ring_gemm_whole_tile_rounds_then_stream_k(dev, bits):
 @pytest.mark.parametrize("splits", [2, 5])
 def test_ring_gemm_forced_split_counts(dev, splits):
     """The gemm_splits override shares every tile among about `splits`
-    workgroups; results equal the default plan's within fp32 rounding and
-    the oracle's within the GEMM tolerance."""
+    workgroups; results equal the default plan's within the rounding of fp16
+    partials and the oracle's within the GEMM tolerance."""
     import ctypes as C
     import r4q_lib as R
     M, N, K = 512, 1280, 4096
@@ -284,60 +285,51 @@ def test_ring_gemm_forced_split_counts(dev, splits):
     assert rel_l2(got, O.gemm(x.numpy(), w.numpy(), sz.numpy(), 4)) <= TOL
 
 
-def _spec(fn):
-    """Runs fn with the specialised-wave GEMM kernel selected."""
+def _plan(M, N, K, bits, ws=0):
+    """(tile rows, tile columns, whole tiles, stream-K workgroups)."""
     import r4q_lib as R
-    R.tune("gemm_kernel", 2)
-    try:
-        return fn()
-    finally:
-        R.tune("gemm_kernel", 0)
+    v = (C.c_int32 * 4)()
+    R.call("r4q_gemm_plan", M, N, K, bits, ws, v, 4)
+    return tuple(v)
+
+
+def _gemm_whole(x, w, sz, M, N, K, bits):
+    """The product without a workspace: whole tiles."""
+    import r4q_lib as R
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device=x.device)
+    R.call("r4q_gemm", x.data_ptr(), w.data_ptr(), None if sz is None else sz.data_ptr(),
+           y.data_ptr(), M, N, K, bits, R.stream_handle())
+    return y
 
 
 @pytest.mark.parametrize("M,N,K", [(512, 17408, 5120), (512, 5120, 17408), (600, 256, 4096),
                                    (512, 7168, 5120), (300, 1280, 2048)])
-def test_spec_gemm_vs_oracle_and_ring(dev, M, N, K):
-    """The specialised-wave kernel (INT4, N % 128 == 0, K % 256 == 0): config
-    3 shapes, a ragged M and split-K shapes against the oracle, and against
-    the ring kernel within fp32 / fp16-partial rounding."""
+def test_tile_gemm_vs_oracle_and_smaller_tiles(dev, M, N, K):
+    """INT4 prompt shapes, a ragged M and split-K shapes against the oracle; in
+    whole 256 x 256 tiles an output is one chain over k, so the first 255 rows
+    alone, which take smaller tiles, give the same bits."""
     g = S.gen(M + 5 * N + K)
     w, sz = S.int4_weight(N, K, g)
     x = torch.randn(M, K, generator=g).half()
     X, Wd, SZ = x.to(dev), w.to(dev), sz.to(dev)
-    ring = int4_hip.dbg_gemm(X, Wd, SZ, M, N, K).float().cpu().numpy()
-    got = _spec(lambda: int4_hip.dbg_gemm(X, Wd, SZ, M, N, K)).float().cpu().numpy()
+    got = int4_hip.dbg_gemm(X, Wd, SZ, M, N, K).float().cpu().numpy()
     assert np.all(np.isfinite(got))
-    assert rel_l2(got, ring) <= 1e-3
     want = _ref32(x, w, sz, 4) if N * K > 4e7 else O.gemm(x.numpy(), w.numpy(), sz.numpy(), 4)
     assert rel_l2(got, want) <= TOL
     for r in (0, M // 2, M - 1):
         assert rel_l2(got[r], want[r]) <= TOL, r
-
-
-def test_spec_gemm_whole_tiles_bit_identical_to_ring(dev):
-    """With whole tiles only (gemm_splits 1) every output element sees the same
-    MFMA sequence in both kernels: bit-identical results."""
-    import r4q_lib as R
-    M, N, K = 512, 1024, 2048
-    g = S.gen(123)
-    w, sz = S.int4_weight(N, K, g)
-    x = torch.randn(M, K, generator=g).half()
-    X, Wd, SZ = x.to(dev), w.to(dev), sz.to(dev)
-    R.tune("gemm_splits", 1)
-    try:
-        ring = int4_hip.dbg_gemm(X, Wd, SZ, M, N, K).cpu().numpy()
-        got = _spec(lambda: int4_hip.dbg_gemm(X, Wd, SZ, M, N, K)).cpu().numpy()
-    finally:
-        R.tune("gemm_splits", 0)
-    assert np.array_equal(got.view(np.uint16), ring.view(np.uint16))
+    assert _plan(M, N, K, 4)[:2] == (256, 256) and _plan(255, N, K, 4)[0] <= 128
+    whole = _gemm_whole(X, Wd, SZ, M, N, K, 4)
+    few = _gemm_whole(X[:255].contiguous(), Wd, SZ, 255, N, K, 4)
+    assert torch.equal(few.view(torch.int16), whole[:255].view(torch.int16))
 
 
 @pytest.mark.parametrize("splits", [0, 3])
-def test_spec_gemm_one_hot_columns_exact(dev, splits):
+def test_tile_gemm_one_hot_columns_exact(dev, splits):
     """Row r of x = e_k(r): y[r] is column k(r) of the dequantised weight, bit
-    for bit, through the specialised-wave kernel's B stages -- in the default
-    plan and with every tile shared by about 3 workgroups (fp16 partials of
-    zeros and one exact product, summed by its reduce)."""
+    for bit -- in the default plan and with every tile shared by about 3
+    workgroups (fp16 partials of zeros and one exact product, summed by the
+    reduce)."""
     import r4q_lib as R
     g = S.gen(211 + splits)
     M, N, K = 300, 384, 2048
@@ -349,11 +341,43 @@ def test_spec_gemm_one_hot_columns_exact(dev, splits):
         x[r, k] = 1.0
     R.tune("gemm_splits", splits)
     try:
-        y = _spec(lambda: int4_hip.dbg_gemm(x.to(dev), w.to(dev), sz.to(dev), M, N, K)).cpu().numpy()
+        y = int4_hip.dbg_gemm(x.to(dev), w.to(dev), sz.to(dev), M, N, K).cpu().numpy()
     finally:
         R.tune("gemm_splits", 0)
     for r, k in enumerate(ks):
         assert np.array_equal(y[r], W[:, k]), (r, k)
+
+
+# (M, N, tile) that the rule takes to each tile of 17 .. 255 rows; N ragged
+TILES = [(31, 4003, (32, 64)), (47, 8259, (48, 64)), (63, 8259, (64, 64)), (64, 16500, (64, 128)),
+         (95, 16500, (96, 128)), (127, 16502, (128, 128)), (200, 34810, (128, 128))]
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16])
+@pytest.mark.parametrize("M,N,tile", TILES)
+def test_every_tile_of_17_to_255_rows(dev, bits, M, N, tile):
+    """Each tile shape in each format, on shapes that the rule takes there, K
+    several times round the ring (17 x 128 + 32, 34 x 64 + 32 k) with a partial
+    last step: against fp32 sums (fp16 output rounding 2.9e-4 rel-L2), and the
+    same bits as its first 17 rows alone, which take 32 x 64 tiles."""
+    K = 2208
+    if bits == 16 and tile[0] == 48:
+        tile = (64, 64)  # 48 x 64 does not exist for FP16 weights
+    assert _plan(M, N, K, bits) == (*tile, -(-M // tile[0]) * -(-N // tile[1]), 0)
+    assert _plan(17, N, K, bits)[:2] == (32, 64)
+    g = S.gen(M + N + bits)
+    w, sz = S.weight(N, K, bits, g)
+    x = torch.randn(M, K, generator=g).half().to(dev)
+    wd, sd = w.to(dev), None if sz is None else sz.to(dev)
+    W = wd if bits == 16 else (int4_hip.dequant_int4 if bits == 4 else int4_hip.dequant_int8)(
+        wd, sd, N, K)
+    want = x.float() @ W.float().T
+    y = int4_hip.dbg_gemm(x, wd, sd, M, N, K)
+    assert torch.isfinite(y).all()
+    err = (y.float() - want).norm(dim=1) / want.norm(dim=1)
+    assert err.max().item() <= 6e-4, err.argmax().item()
+    few = int4_hip.dbg_gemm(x[:17].contiguous(), wd, sd, 17, N, K)
+    assert torch.equal(few.view(torch.int16), y[:17].view(torch.int16))
 
 
 @pytest.mark.parametrize("bits", [4, 8, 16])
@@ -362,23 +386,21 @@ def test_spec_gemm_one_hot_columns_exact(dev, splits):
                                    (128, 20000, 96), (129, 1000, 1312), (255, 383, 4192),
                                    (256, 257, 1056), (257, 70, 96), (513, 1030, 2080)])
 def test_tile_gemm_edges(dev, bits, M, N, K):
-    """M > 16: one row past and one short of every tile height, widths off the
-    tile and off the 16-byte store, K shorter than a step and ending inside one,
+    """32 x 64 tiles (narrow N takes every M below 256 there; 128 x 20000: 128 x
+    128) and 256 x 256 ones: rows and widths one past and one short of a tile,
+    widths off the 16-byte store, K shorter than a step and ending inside one,
     split and unsplit (no workspace).  The fp16 output rounds within 2^-12
     relative (rel-L2 below 2.9e-4), a fp16 partial (M >= 256) as much again per
     segment: 1e-3 is twice their sum over the at most 16 segments' random
-    signs.  Below 256 rows an output is one chain over k in any tile, so rows
-    alone in a smaller tile (their first 17) give the same bits."""
-    import r4q_lib as R
+    signs.  In whole tiles an output is one chain over k, so rows alone in a
+    smaller tile (their first 17) give the same bits."""
     g = S.gen(M + 7 * N + K + bits)
     w, sz = S.weight(N, K, bits, g)
     x = torch.randn(M, K, generator=g).half()
     X, Wd, SZ = x.to(dev), w.to(dev), None if sz is None else sz.to(dev)
     want = _ref32(x, w, sz, bits)
     split = int4_hip.dbg_gemm(X, Wd, SZ, M, N, K)
-    whole = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
-    R.call("r4q_gemm", X.data_ptr(), Wd.data_ptr(), None if SZ is None else SZ.data_ptr(),
-           whole.data_ptr(), M, N, K, bits, R.stream_handle())
+    whole = _gemm_whole(X, Wd, SZ, M, N, K, bits)
     for y in (split, whole):
         got = y.float().cpu().numpy()
         assert np.all(np.isfinite(got))
@@ -387,8 +409,6 @@ def test_tile_gemm_edges(dev, bits, M, N, K):
             assert rel_l2(got[r], want[r]) <= 1e-3, r
     few = int4_hip.dbg_gemm(X[:17].contiguous(), Wd, SZ, 17, N, K)
     assert torch.equal(few.view(torch.int16), whole[:17].view(torch.int16))
-    if M < 256:
-        assert torch.equal(split.view(torch.int16), whole.view(torch.int16))
 
 
 @pytest.mark.parametrize("bits", [4, 8, 16])
@@ -418,14 +438,17 @@ def test_tile_gemm_one_hot_and_infinite_rows(dev, bits, M, N, K):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("M,N,K", [(17, 70, 1056), (48, 8259, 352), (64, 8259, 1184), (64, 16500, 608),
-                                   (96, 16500, 736), (128, 16500, 352), (255, 300, 2080)])
-def test_tile_gemm_zero_points_of_any_value(dev, bits, M, N, K):
+@pytest.mark.parametrize("M,N,K,tile", [
+    (17, 70, 1056, (32, 64)), (48, 8259, 352, (48, 64)), (64, 8259, 1184, (64, 64)),
+    (64, 16500, 608, (64, 128)), (96, 16500, 736, (96, 128)), (128, 16500, 352, (128, 128)),
+    (255, 300, 2080, (32, 64))])
+def test_tile_gemm_zero_points_of_any_value(dev, bits, M, N, K, tile):
     """fp16((q - zp) * scale) holds for every zero-point below 256 rows, whole
-    number or not, in every tile shape (32 x 64 .. 128 x 128 in this order):
-    row r of x = e_k(r) gives column k(r) of the oracle's dequantised weight bit
-    for bit where blocks with other zero-points sit among the usual ones, in
-    some weight rows only, and in a last partial step."""
+    number or not, in every tile shape: row r of x = e_k(r) gives column k(r) of
+    the oracle's dequantised weight bit for bit where blocks with other
+    zero-points sit among the usual ones, in some weight rows only, and in a
+    last partial step."""
+    assert _plan(M, N, K, bits)[:2] == tile
     g = S.gen(3 * M + N + K + bits)
     w, sz = S.weight(N, K, bits, g)
     z = sz.view(N, K // 32, 2)[:, :, 1]
