@@ -446,9 +446,9 @@ struct TileSeg {
   // the first wait stricter (copies retire in order among themselves).
   // kAnyZp: a tile with zero-points that dqp rounds is computed again, with dqx:
   // 96 x 7168 x 5120 INT4 21 us, with such zero-points 51.  The look costs 96 x 7168 x
-  // 5120 20.7 -> 21.3, 64 x 5120 x 17408 52.8 -> 56.4, 128 x 34816 x 5120 79.5 -> 81.3;
-  // a branch in every step took the first two to 25.2 and 62.8, a fifth wave that
-  // looks all three to 23.1, 57.1 and 98.6.
+  // 5120 20.5 -> 21.2, 64 x 5120 x 17408 52.5 -> 56.2, 128 x 34816 x 5120 77.6 -> 79.2
+  // (INT8: 20.3 -> 20.9, 51.3 -> 50.5, nothing); a branch in every step took the first
+  // two to 25.2 and 62.8, a fifth wave that looks all three to 23.1, 57.1 and 98.6.
   __device__ __forceinline__ void run(f4_t (&acc)[NF][MT], int t) const {
     Zp zp;
     loop(acc, t, zp);
@@ -509,11 +509,18 @@ struct TileSeg {
       ring_barrier();
       if (tail && i + 1 == nk) clear_tail(nk - 1, cur, t);
       load_raw(cur, raw);
+      // the word to look at: read ahead of the X fragments or after them, as the
+      // compiled loop measured faster (us ahead / after: 17 x 7168 x 5120 INT8 17.4 / 18.5,
+      // INT4 20.9 / 19.0, 128 x 5120 x 17408 INT8, 48-row tiles, 57.3 / 55.3), and
+      // looked at in the next step, when it is there
+      constexpr bool kAhead = WBITS == 8 && NF == 1 && MT != 3;
+      uint32_t zn = 0;
+      if constexpr (kAnyZp && kAhead) zn = zp_word(cur);
 #pragma unroll
       for (int q = 0; q < T::P; ++q) a[q] = xfrag(cur, q);
-      if constexpr (kAnyZp) {  // (at the word of the step before: it is there)
+      if constexpr (kAnyZp) {
         zp.look(zw);
-        zw = zp_word(cur);
+        zw = kAhead ? zn : zp_word(cur);
       }
 #pragma unroll
       for (int f = 0; f < NF; ++f) b[f] = dq(raw, f, 0);
