@@ -15,9 +15,10 @@ namespace {
 
 // Eight consecutive elements (16 bytes of fp16) per thread and turn: loads and
 // stores of a wave are contiguous.  kTurns turns of a workgroup apart, so that
-// several loads are in flight.  Bound by HBM, 7/8 of it writes at INT4: 17408 x
-// 5120 INT4 61 -> 35 us (6.6 TB/s), INT8 67 -> 43; before, a 32-element block per
-// thread wrote 16 bytes of every 64 per store instruction.
+// several loads are in flight.  Bound by HBM, three quarters of it writes at INT4
+// (2 of 2.625 bytes per element): 17408 x 5120 INT4 61 -> 35 us (6.6 TB/s), INT8 67 ->
+// 43; before, a 32-element block per thread wrote 16 bytes of every 64 per store
+// instruction.
 constexpr int kTurns = 4;
 template <int WBITS>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ w,

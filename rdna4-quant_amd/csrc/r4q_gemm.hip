@@ -147,16 +147,24 @@ __device__ __forceinline__ int sk_owner(int64_t u, int64_t TU, int sk) {
 // of the TU = (T - dp) U flattened ones.  A tile shared by several workgroups
 // gets one fp16 partial per workgroup (segment), summed in fp32 in segment
 // order by gemm_tile_reduce_kernel: the result does not depend on timing.
-// What bounds it: M >= 256, MFMA issue: at 512 x 32768 x 5120 INT4 the matrix
-// cores are busy 48% of the cycles at the 2.0 GHz (of 2.4) that the power limit
-// leaves; 57% without the dequantisation, unchanged without the copies.  M <
-// 256, the serial chain of K steps (0.34 us per 128 k for a 32 x 64 tile).
-// Measured (us, before: a 128 x 128 kernel with one 32-wide step in flight for
-// M < 256, 256 x 256 tiles with one wave per SIMD for M >= 256): INT4 17 x 7168 x
-// 5120 118 -> 19, 96 x 7168 x 5120 124 -> 22, 128 x 5120 x 17408 421 -> 63, 255 x 4192 x
-// 383 INT8 106 -> 16, 24 x 151936 x 5120 FP16 395 -> 283; 512 x 17408 x 5120 INT4
-// 126 -> 120, 512 x 5120 x 17408 118 -> 109, 512 x 34816 x 5120 210 -> 196, 1999 x 34816 x
-// 5120 INT8 725 -> 686 (1.04 PFLOP/s), 512 x 151936 x 5120 FP16 953 -> 784.
+// What bounds it: M >= 256, the work of a step that its MFMAs do not cover: at 512 x
+// 32768 x 5120 INT4 the matrix cores are busy 48% of the cycles at the 2.0 GHz (of
+// 2.4) that the power limit leaves, 57% without the dequantisation.  Timing
+// builds of that shape, us with everything / without the copies / without the
+// steps' barriers too: INT4 160 / 144 / 133, INT8 158 / 148 / 135, FP16 (2 stages,
+// every step opens with a wait for its copies) 163 / 121 / 119 -- on what the LDS
+// happens to hold, which also draws less power.  The rest, the LDS reads and the
+// dequantisation ahead of a step's first MFMA among it, is not taken apart.
+// M < 256, the serial chain of K steps (0.34 us per 128 k for a 32 x 64 tile),
+// whose parts are not taken apart either.
+// Measured (us, graph replays on one box, weights not evicted between them;
+// before: a 128 x 128 kernel with one 32-wide step in flight for M < 256, 256 x
+// 256 tiles with one wave per SIMD for M >= 256): INT4 17 x 7168 x 5120 116 -> 20,
+// 96 x 7168 x 5120 122 -> 23, 128 x 5120 x 17408 420 -> 71, 96 x 34816 x 5120 139 -> 70,
+// 24 x 151936 x 5120 FP16 396 -> 282; 512 x 17408 x 5120 INT4 126 -> 112, 512 x 5120 x
+// 17408 109 -> 102, 512 x 34816 x 5120 198 -> 187, 1999 x 34816 x 5120 INT8 796 -> 707 (1.01
+// PFLOP/s), 512 x 151936 x 5120 FP16 958 -> 804.  Another box, and less heat, moves
+// them by up to 15%.
 template <int WBITS, int MT, int NF, int MG>
 struct Tile {
   static constexpr int kMG = MG;
@@ -754,7 +762,7 @@ __global__ __launch_bounds__(256) void gemm_tile_reduce_kernel(const uint16_t* _
 // LDS then allows it); one barrier per step
 // (the ring of gemm_tile_kernel).  Per step each wave runs KS/32 MFMA
 // 16x16x32 tiles: B = its 16 weight rows dequantised from LDS (skinny_b),
-// A = the activation rows (skinny_a's element order), C = 16 activation
+// A = the activation rows (in the k labels below), C = 16 activation
 // rows x 16 weight rows.  Lane group g of MFMA j holds the k labels
 // k0 + (KS/4) g + 8 j .. +7 in both operands, so each lane reads its 32
 // weight bytes of the step with two 16-byte LDS reads.  The 16-byte pieces
@@ -1360,7 +1368,9 @@ struct TilePlan {
   size_t ws = 0;  // partials: (tiles - dp) * maxseg tiles
 };
 
-constexpr int kTileCUs = 256;  // MI355X compute units: one tile workgroup each (LDS-bound)
+// MI355X compute units.  Their LDS holds one workgroup of a 256 x 256 tile, two of
+// the others.
+constexpr int kTileCUs = 256;
 
 // Host restatement of sk_lo / sk_owner (the kernel's unit split).
 static int64_t host_sk_lo(int64_t w, int64_t TU, int64_t sk) { return w * TU / sk; }
@@ -1422,13 +1432,18 @@ static TilePlan split_plan(int64_t tiles, int U, int64_t tile_bytes, size_t ws_b
   return pl;
 }
 
-// Tile shape.  M >= 256: 256 x 256, the K of its tiles split (32-bit byte offsets
-// cover its rows; operands of 4 GiB and more take the shapes below).
+// Tile shape.  M >= 256: 256 x 256, the K of its tiles split.  Operands of 4 GiB and
+// more take the shapes below, in whole tiles, as they did before there were tiles
+// of 256 rows: the copies would allow more (their 32-bit offsets count from the
+// tile's first row), but fp16 partials would round what is not rounded now.
 // M < 256 (and those): whole tiles over all of K, one fp32 chain per output,
 // so the tile decides how many CUs work.  The time follows the most loaded
 // CU, ceil(tiles / 256) x the time of a tile's K step, which hardly depends on
-// how many tiles of a shape share the CU; measured per 128 k (us): 32 x 64 0.34,
-// 48 x 64 0.40, 64 x 64 0.45, 64 x 128 0.88, 96 x 128 0.98, 128 x 128 1.15.  E.g.
+// how many tiles of a shape share the CU; measured at INT4 per 128 k (us): 32 x 64
+// 0.34, 48 x 64 0.40, 64 x 64 0.45, 64 x 128 0.88, 96 x 128 0.98, 128 x 128 1.15.  INT8
+// and FP16 steps copy more bytes of weights; no table of their own was measured,
+// but on 13 row counts from 17 to 255 and 8 widths the choice was 1.2 to 7 times as
+// fast as the 128 x 128 kernel before it in every format.  E.g.
 // (us) 96 x 7168 x 5120 INT4 29 / 22 / 24 / 41 / 47 / 52 over those shapes, 96 x 34816 x
 // 5120 98 / 83 / 91 / 104 / 84 / 87, 96 x 5120 x 17408 INT8 58 / 73 / 73 / 138 / 174 / 174,
 // 200 x 34816 x 5120 195 / 169 / 156 / 166 / 150 / 141.

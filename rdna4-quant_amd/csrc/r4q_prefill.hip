@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256) void embed_gather_kernel(const int64_t* __rest
 // lane, steps 1 .. 8 across lanes xor 1 .. 8), one fp16 rounding.
 //
 // Bound by the softmax's vector instructions with the waves that one CU holds (four
-// workgroups, 128 VGPRs).  40 heads over 8 K/V heads, 2000 rows: 207 -> 82 us; 512
+// workgroups, 128 VGPRs).  40 heads over 8 K/V heads, 2000 rows: 191 -> 76-79 us; 512
 // rows: 31 -> 19 us, a chain of 16 turns in the longest workgroup.  Before, V was
 // transposed by 2-byte LDS stores that conflicted 4 ways, K, softmax and V of a
 // block were one chain, and the tiles with the fewest keys came first.  32 query
