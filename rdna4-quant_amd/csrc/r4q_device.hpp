@@ -345,7 +345,8 @@ __device__ __forceinline__ uint32_t lds_off(const lds8* p) {
 
 // Global -> LDS copies of 16 (4) bytes per lane: lane l's bytes land at
 // lds + 16 l (4 l).  copy16s / copy4s: a uniform 64-bit base and a 32-bit byte
-// offset per lane; copy16: an address per lane.  Inline assembly, so that the
+// offset per lane, OFF bytes on from lds (the sum goes to m0 in one instruction);
+// copy16: an address per lane.  Inline assembly, so that the
 // compiler's wait counts do not see the copies: it would otherwise wait for every
 // copy in flight before any LDS read; the kernels wait for their own copies.  The
 // hardware takes the LDS address from m0 (one wait state after its write), which
@@ -353,15 +354,29 @@ __device__ __forceinline__ uint32_t lds_off(const lds8* p) {
 // each of its own uses, of which a kernel with these copies should have none.
 // The base has to come from scalar arithmetic: written by a vector instruction
 // it would need five wait states.
+template <int OFF = 0>
 __device__ __forceinline__ void copy16s(const void* base, uint32_t off, lds8* lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_off(lds)),
-               "v"(off), "s"(base)
-               : "memory");
+  if constexpr (OFF == 0)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_off(lds)),
+                 "v"(off), "s"(base)
+                 : "memory");
+  else
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
+                     lds_off(lds)),
+                 "v"(off), "s"(base), "n"(OFF)
+                 : "memory", "scc");
 }
+template <int OFF = 0>
 __device__ __forceinline__ void copy4s(const void* base, uint32_t off, lds8* lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_off(lds)),
-               "v"(off), "s"(base)
-               : "memory");
+  if constexpr (OFF == 0)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_off(lds)),
+                 "v"(off), "s"(base)
+                 : "memory");
+  else
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(
+                     lds_off(lds)),
+                 "v"(off), "s"(base), "n"(OFF)
+                 : "memory", "scc");
 }
 __device__ __forceinline__ void copy16(const void* src, lds8* lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_off(lds)),

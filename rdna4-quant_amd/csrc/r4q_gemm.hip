@@ -291,15 +291,28 @@ struct TileSeg {
                st + 1024 * T::CX * wave, st + T::kX + 1024 * T::CW * wave,
                st + T::kX + T::kW + 256 * T::CS * wave};
   }
-  __device__ __forceinline__ void copy(const Src& s, int c) const {
-    if (c < T::CX) copy16s(s.x, xo[c], s.dx + 1024 * c);
-    else if (c < T::CX + T::CW) copy16s(s.w, wo[c - T::CX], s.dw + 1024 * (c - T::CX));
-    else copy4s(s.s, so[c - T::CX - T::CW], s.ds + 256 * (c - T::CX - T::CW));
+  // (offsets added in the copy's own instruction below 256 rows: 0-3% faster there,
+  // 1999 x 34816 x 5120 INT8 1% slower)
+  template <int C>
+  __device__ __forceinline__ void copy(const Src& s) const {
+    constexpr bool kX = C < T::CX, kW = !kX && C < T::CX + T::CW;
+    constexpr int kOff = kX ? 1024 * C : kW ? 1024 * (C - T::CX) : 256 * (C - T::CX - T::CW);
+    constexpr int kIn = MG == 1 ? kOff : 0, kOut = kOff - kIn;
+    if constexpr (kX) copy16s<kIn>(s.x, xo[C], s.dx + kOut);
+    else if constexpr (kW) copy16s<kIn>(s.w, wo[C - T::CX], s.dw + kOut);
+    else copy4s<kIn>(s.s, so[C - T::CX - T::CW], s.ds + kOut);
+  }
+  // the copies c >= C for which f(c)
+  template <int C = 0, class F>
+  __device__ __forceinline__ void copies(const Src& s, F f) const {
+    if constexpr (C < T::kPer) {
+      if (f(C)) copy<C>(s);
+      copies<C + 1>(s, f);
+    }
   }
   __device__ __forceinline__ void issue(int i, lds8* st) const {
     const Src s = src(i, st);
-#pragma unroll
-    for (int c = 0; c < T::kPer; ++c) copy(s, c);
+    copies(s, [](int) { return true; });
   }
 
   // zeroes what the stage of a last step i holds outside its own k (before
@@ -453,10 +466,12 @@ struct TileSeg {
   // the segment's K loop, after start(); stores issued since then only make
   // the first wait stricter (copies retire in order among themselves).
   // kAnyZp: a tile with zero-points that dqp rounds is computed again, with dqx:
-  // 96 x 7168 x 5120 INT4 21 us, with such zero-points 51.  The look costs 96 x 7168 x
-  // 5120 20.5 -> 21.2, 64 x 5120 x 17408 52.5 -> 56.2, 128 x 34816 x 5120 77.6 -> 79.2
-  // (INT8: 20.3 -> 20.9, 51.3 -> 50.5, nothing); a branch in every step took the first
-  // two to 25.2 and 62.8, a fifth wave that looks all three to 23.1, 57.1 and 98.6.
+  // 96 x 7168 x 5120 INT4 21 us, with such zero-points 51.  Without the look / with it,
+  // us: 96 x 7168 x 5120 INT4 20.6 / 21.0, 64 x 5120 x 17408 52.3 / 53.9, 128 x 34816 x 5120
+  // 78.3 / 81.3; INT8 18.9 / 19.6, 51.5 / 48.2, 255 x 34816 x 5120 133 / 132 (with the copies'
+  // LDS addresses taken in one instruction, which gave 0-3% back).  A branch in every
+  // step took the first two to 25.2 and 62.8, a fifth wave that looks the first three
+  // to 23.1, 57.1 and 98.6.
   __device__ __forceinline__ void run(f4_t (&acc)[NF][MT], int t) const {
     Zp zp;
     loop(acc, t, zp);
@@ -517,19 +532,18 @@ struct TileSeg {
       ring_barrier();
       if (tail && i + 1 == nk) clear_tail(nk - 1, cur, t);
       load_raw(cur, raw);
-      // the word to look at: read ahead of the X fragments or after them, as the
-      // compiled loop measured faster (us ahead / after: 17 x 7168 x 5120 INT8 17.4 / 18.5,
-      // INT4 20.9 / 19.0, 128 x 5120 x 17408 INT8, 48-row tiles, 57.3 / 55.3), and
-      // looked at in the next step, when it is there
-      constexpr bool kAhead = WBITS == 8 && NF == 1 && MT != 3;
+      // the word to look at, read ahead of the X fragments or after them, and looked
+      // at in the next step or in this one's last MFMAs, as measured: us of 17 x 7168 x
+      // 5120 INT4 next / this step 18.8 / 18.2, INT8 ahead 17.0, after them 17.7; 128 x
+      // 5120 x 17408 (48-row tiles) INT4 61.0 / 63.8, INT8 ahead 57.3, after them 55.3
+      constexpr bool kTuned = kAnyZp && NF == 1 && MT != 3;
+      constexpr bool kAhead = kTuned && WBITS == 8, kLate = kTuned && WBITS == 4;
       uint32_t zn = 0;
-      if constexpr (kAnyZp && kAhead) zn = zp_word(cur);
+      if constexpr (kAhead) zn = zp_word(cur);
 #pragma unroll
       for (int q = 0; q < T::P; ++q) a[q] = xfrag(cur, q);
-      if constexpr (kAnyZp) {
-        zp.look(zw);
-        zw = kAhead ? zn : zp_word(cur);
-      }
+      if constexpr (kAnyZp && !kLate) zp.look(zw);
+      if constexpr (kAnyZp) zw = kAhead ? zn : zp_word(cur);
 #pragma unroll
       for (int f = 0; f < NF; ++f) b[f] = dq(raw, f, 0);
       const Src sc0 = src(i + T::D - 1, far);
@@ -543,13 +557,18 @@ struct TileSeg {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
           const int q = j * MT + m;
-#pragma unroll
-          for (int c = 0; c < T::kPer; ++c)
-            if (c * T::Q / T::kPer == q) copy(sc0, c);
+          copies(sc0, [q](int c) { return c * T::Q / T::kPer == q; });
 #pragma unroll
           for (int f = 0; f < NF; ++f)
             acc[f][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[f], a[q % T::P], acc[f][m], 0, 0, 0);
           if (q + T::P < T::Q) a[q % T::P] = xfrag(cur, q + T::P);
+          if constexpr (kLate) {
+            if (q == T::Q - 2) {
+              asm volatile("" : "+v"(zw));  // not earlier
+              zp.look(zw);
+              zw = 0;
+            }
+          }
 #pragma unroll
           for (int e = m * 4 * NF / MT; e < (m + 1) * 4 * NF / MT; ++e) {
             if (j + 1 < T::J) bn[e / 4][e % 4] = dqp(raw, e / 4, j + 1, e % 4, nz, sc, w4);
